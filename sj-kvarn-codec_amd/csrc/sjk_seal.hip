@@ -18,9 +18,12 @@
 //   * quantize (sj_kvarn.h:1112-1147): row min/max (ordered chunk combine, NaN-exact), then one thread
 //     per 8 codes writes b bytes of payload (4-bit fragment order, token-major or channel-major);
 //   * trellis (sj_kvarn.h:1025-1109): one wavefront per channel runs the 64-state Viterbi with one
-//     state per lane (path metrics exchanged with ds_bpermute, branch choices packed in registers,
+//     state per lane (sums on the matrix unit, path metrics exchanged with ds_bpermute, choices packed in registers,
 //     traceback with readlane), then one thread per row does the moment-matching refit.
 #include "sjk_dev.h"
+
+#include <type_traits>
+#include <utility>
 
 namespace sjk {
 
@@ -386,51 +389,127 @@ SJK_DEV void col_scales(const SealArgs & a, SealLds & s, uint8_t * rec) {
 
 SJK_DEV float readlane_f(float x, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane)); }
 
-// 64-state Viterbi of one channel, one state per lane (sj_kvarn.h:1025-1053). y0/y1: target of token
-// lane / lane + 64. Returns the codes of tokens lane and lane + 64.
-template <int BITS>
-SJK_DEV void viterbi_wave(float y0, float y1, const float * cbf, int lane, uint32_t & c0, uint32_t & c1) {
-    constexpr int NB = 1 << BITS;
-    float cbv[NB];
-    int src[NB];
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+// p = 2 p + (bit `lane` of m), one instruction. m must come from the scalar unit (a mask straight from a vector
+// compare needs two wait states before a vector instruction reads it, which the compiler does not insert for asm).
+SJK_DEV uint32_t shift_in(uint32_t p, uint64_t m) {
+    uint32_t r;
+    asm("v_addc_co_u32_e64 %0, vcc, %1, %1, %2" : "=v"(r) : "v"(p), "s"(m) : "vcc");
+    return r;
+}
+
+// lane I of v = x (uniform)
+template <int I> SJK_DEV void set_lane(uint32_t & v, uint32_t x) {
+    asm("v_writelane_b32 %0, %1, %2" : "+v"(v) : "s"(x), "n"(I));
+}
+
+// f(0), ..., f(N - 1) with constant arguments
+template <typename F, int... I> SJK_DEV void for_const(F && f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+
+SJK_DEV uint64_t lanes_eq(uint32_t a, uint32_t b) { return __builtin_amdgcn_ballot_w64(a == b); }
+SJK_DEV uint32_t umin3(uint32_t a, uint32_t b, uint32_t c) { return min(min(a, b), c); }
+
+// 64-state Viterbi of one channel, one state per lane (sj_kvarn.h:1025-1053): M'[s] = min_j (y - cb[s + 64 j])^2 +
+// M[(s + 64 j) >> BITS], the first j on a tie (the reference's strict <). y[h]: target of token lane + 64 h; returns
+// the codes of the same tokens. What bounds it: the 512 branches of a step are 8 costs a lane, whose predecessor
+// metrics by ds_bpermute (8 a step at 6 LDS cycles each, 16 wavefronts a CU: 770 cycles a step of all of them) and
+// compare / select / index chains held the plain form at about 900 cycles a step of the four wavefronts of a SIMD
+// (0.92 ms per 4096-token 3/2 commit). So both are moved to the matrix and the scalar unit:
+//   * y - cb and e + M: v_mfma_f32_4x4x1 is D[i] = RN(A x B + C) per lane with one product, so with B = 1 it is the
+//     correctly rounded sum, subnormals included (checked on the device over random operands), four values a lane
+//     per instruction beside the vector unit. Row i is branch 4 t + i. For y - cb, C = -cb and A = y of the token: the
+//     16 tokens of a block sit in the 16 blocks of four lanes, and the instruction's block broadcast picks one. For
+//     e + M, row i of a lane's block of four is the predecessor metric of branch 4 t + i, which its four lanes share
+//     (2^BITS / 4 ds_bpermute a step instead of 2^BITS);
+//   * the costs are >= +0 and finite, so their bits order like the floats: the minimum is v_min3_u32, the branch
+//     taken is the first that equals it, worked out as lane masks on the scalar unit and shifted into the picks one
+//     bit an instruction.
+// 24 vector + 4 matrix instructions and 2 permutes a step at 3 bits (13 + 2 and 1 at 2 bits), about 670 cycles a step
+// of the four wavefronts: 0.72 ms per 4096-token 3/2 commit. The picks cost 260 of them and the squares, minima and
+// matrix instructions the rest; two channels in one loop or y - cb on the vector unit are no faster (0.73, 0.76 ms).
+// The loop takes 32 tokens, so that the code of both sides stays in the instruction cache; the picks of the last 32
+// tokens enter at the end of pk, which moves up.
+// XN: a side that holds an infinity or a NaN. The reference starts from +inf and takes a branch only when its cost is
+// below, so that infinite and NaN costs never win and branch 0 stays: such costs are clamped to +inf (a NaN's bits
+// are above it, of either sign), where they all tie.
+template <int BITS, bool XN>
+SJK_DEV void viterbi_wave(const float (&y)[2], const float * cbf, int lane, uint32_t (&code)[2]) {
+    constexpr int NB = 1 << BITS, NT = NB / 4;       // branches, and 4-branch tuples
+    constexpr int SPW = BITS == 3 ? 8 : 16;          // steps per word of picks
+    constexpr int WPL = 32 / SPW, NW = 4 * WPL;      // words of picks per 32 tokens, per channel
+    f4 ncb[NT];
+    int src[NT];                                     // lane (x 4) of the predecessor of branch 4 t + (lane & 3)
 #pragma unroll
-    for (int j = 0; j < NB; ++j) {
-        cbv[j] = cbf[lane + 64 * j];
-        src[j] = ((lane + 64 * j) >> BITS) * 4;
+    for (int t = 0; t < NT; ++t) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ncb[t][i] = -cbf[lane + 64 * (4 * t + i)];
+        src[t] = 4 * (((lane & ~3) + 64 * (4 * t + (lane & 3))) >> BITS);
     }
-    float M = 0.0f;
-    uint32_t picks[16];
+    uint32_t M = 0;                                  // the path metric's bits
+    uint32_t pk[NW];
 #pragma unroll
-    for (int w = 0; w < 16; ++w) picks[w] = 0;
+    for (int q = 0; q < NW; ++q) pk[q] = 0;
+#pragma unroll 1
+    for (int it = 0; it < 4; ++it) {                 // tokens 127 - 32 it down to 96 - 32 it
+        uint32_t w[WPL];
+        float yt;
+        auto step = [&](auto K) {
+            constexpr int k = decltype(K)::value, tk = 31 - k;       // token 96 - 32 it + tk
+            if constexpr (k % 16 == 0)
+                yt = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * (((96 - 32 * it) & 63) + (tk & 16) + (lane >> 2)),
+                                                                 __float_as_int(it < 2 ? y[1] : y[0])));
+            uint32_t x[NB];
 #pragma unroll
-    for (int i = 127; i >= 0; --i) {
-        const float yi = readlane_f(i < 64 ? y0 : y1, i & 63);
-        float best = __builtin_inff();
-        uint32_t pick = 0;
+            for (int t = 0; t < NT; ++t) {
+                const float mp = __int_as_float(__builtin_amdgcn_ds_bpermute(src[t], (int) M));
+                f4 e = __builtin_amdgcn_mfma_f32_4x4x1f32(yt, 1.0f, ncb[t], 4, tk & 15, 0);
+                e = e * e;
+                e = __builtin_amdgcn_mfma_f32_4x4x1f32(mp, 1.0f, e, 0, 0, 0);
 #pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            const float d = yi - cbv[j];
-            const float e = d * d;
-            const float mp = __int_as_float(__builtin_amdgcn_ds_bpermute(src[j], __float_as_int(M)));
-            const float c = e + mp;
-            if (c < best) { best = c; pick = (uint32_t) j; }
-        }
-        M = best;
-        picks[i >> 3] |= pick << (4 * (i & 7));
+                for (int r = 0; r < 4; ++r) x[4 * t + r] = XN ? min(f_bits(e[r]), 0x7F800000u) : f_bits(e[r]);
+            }
+            uint32_t p = k % SPW == 0 ? 0u : w[k / SPW];
+            if constexpr (BITS == 3) {
+                const uint32_t best = min(umin3(umin3(umin3(x[0], x[1], x[2]), x[3], x[4]), x[5], x[6]), x[7]);
+                const uint64_t m0 = lanes_eq(x[0], best), m1 = lanes_eq(x[1], best), m2 = lanes_eq(x[2], best),
+                               m3 = lanes_eq(x[3], best), m4 = lanes_eq(x[4], best), m5 = lanes_eq(x[5], best),
+                               m6 = lanes_eq(x[6], best);
+                const uint64_t m01 = m0 | m1, m23 = m2 | m3;
+                p = shift_in(p, ~(m01 | m23));
+                p = shift_in(p, ~m01 & (m23 | ~(m4 | m5)));
+                p = shift_in(p, ~m0 & (m1 | (~m2 & (m3 | (~m4 & (m5 | ~m6))))));
+                M = best;
+            } else {
+                const uint32_t best = min(umin3(x[0], x[1], x[2]), x[3]);
+                const uint64_t m0 = lanes_eq(x[0], best), m1 = lanes_eq(x[1], best), m2 = lanes_eq(x[2], best);
+                p = shift_in(p, ~(m0 | m1));
+                p = shift_in(p, ~m0 & (m1 | ~m2));
+                M = best;
+            }
+            w[k / SPW] = p;
+        };
+        for_const(step, std::make_integer_sequence<int, 32>{});
+#pragma unroll
+        for (int q = 0; q < NW - WPL; ++q) pk[q] = pk[q + WPL];
+#pragma unroll
+        for (int q = 0; q < WPL; ++q) pk[NW - WPL + q] = w[q];
     }
+    // traceback: word q holds tokens 127 - SPW q down to 128 - SPW (q + 1), the last in the low bits
     int st = 0;
-    c0 = 0; c1 = 0;
-#pragma unroll
-    for (int i = 0; i < 128; ++i) {
-        const int pk = (int) ((uint32_t) __builtin_amdgcn_readlane((int) picks[i >> 3], st) >> (4 * (i & 7))) & 15;
-        if (i < 64) c0 = lane == i ? (uint32_t) pk : c0;
-        else c1 = lane == i - 64 ? (uint32_t) pk : c1;
-        st = (st + 64 * pk) >> BITS;
-    }
+    code[0] = code[1] = 0;
+    for_const([&](auto T) {
+        constexpr int i = decltype(T)::value, q = (127 - i) / SPW, last = 128 - SPW * (q + 1);
+        const uint32_t j = ((uint32_t) __builtin_amdgcn_readlane((int) pk[q], st) >> (BITS * (i - last))) & (NB - 1u);
+        set_lane<(i & 63)>(code[i >> 6], j);
+        st = (st >> BITS) + (int) (j << (6 - BITS));
+    }, std::make_integer_sequence<int, 128>{});
 }
 
 template <int R, int C, bool IS_V, int BITS>
-SJK_DEV void trellis_side(const SealArgs & a, SealLds & s, uint8_t * rec) {
+SJK_DEV void trellis_side(const SealArgs & a, SealLds & s, uint8_t * rec, bool nonfinite) {
     constexpr int D = IS_V ? C : R, G = IS_V ? R : C;
     static_assert(G == 128, "trellis sequences are 128 tokens");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -443,10 +522,11 @@ SJK_DEV void trellis_side(const SealArgs & a, SealLds & s, uint8_t * rec) {
             const int r = IS_V ? t : d, c = IS_V ? d : t;
             y[hh] = (cur_at<C>(s, r, c) - s.qlo[r]) / s.qstep[r];
         }
-        uint32_t c0, c1;
-        viterbi_wave<BITS>(y[0], y[1], s.cbf, lane, c0, c1);
-        s.u.codes[d * 128 + lane] = (uint8_t) c0;
-        s.u.codes[d * 128 + lane + 64] = (uint8_t) c1;
+        uint32_t code[2];
+        if (nonfinite) viterbi_wave<BITS, true>(y, s.cbf, lane, code);
+        else viterbi_wave<BITS, false>(y, s.cbf, lane, code);
+        s.u.codes[d * 128 + lane] = (uint8_t) code[0];
+        s.u.codes[d * 128 + lane + 64] = (uint8_t) code[1];
     }
     __syncthreads();
     // pack channel-major: unit u = 8 tokens of one channel
@@ -523,8 +603,8 @@ SJK_DEV void seal_side(const SealArgs & a, SealLds & s, int il, int g, int h, ui
     }
     if (a.lay.body == SJKVARN_BODY_TRELLIS) {
         const int bits = IS_V ? a.lay.bits_v : a.lay.bits_k;
-        if (bits == 3) trellis_side<R, C, IS_V, 3>(a, s, rec);
-        else trellis_side<R, C, IS_V, 2>(a, s, rec);
+        if (bits == 3) trellis_side<R, C, IS_V, 3>(a, s, rec, nonfinite);
+        else trellis_side<R, C, IS_V, 2>(a, s, rec, nonfinite);
     } else {
         scalar_codes<R, C, IS_V>(a, s, rec);
     }
