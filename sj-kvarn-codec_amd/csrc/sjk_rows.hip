@@ -276,6 +276,119 @@ __global__ void decode_kernel(sj_kvarn_layout l, const uint8_t * body, int n_rec
                          get_half(rec, l.v_zero + 2u * (uint32_t) t), get_half(rec, l.v_ch + 2u * (uint32_t) v_ch_idx(l, d)));
 }
 
+// Decode of records with a layer's own geometry (D = 128 or 256, G = 128) whose words are aligned. The kernel above is
+// bound by its byte loads and address arithmetic, ~60 instructions a value (41 us for 64 3/2 trellis records at D = 256:
+// 18.2 MB, 16.8 of them written). Here a thread makes 4 consecutive channels x 8 tokens of one side: whole words of codes
+// in (four 8-byte reads of the 4-bit order, a channel's 8 codes and history as one 32-bit window of a trellis), one
+// 16-byte store per token out; the trellis codebook sits in LDS as floats. 9.3 us for the
+// same records, of which the launch is ~4; a first form of 12 us converted the halves with f16_to_f32's branches.
+// The values are those of dequant_x: the plain products and sum unless the result is a NaN, whose sign dequant_x gives
+// (a NaN made on the way stays one, so checking the result is enough).
+SJK_DEV float dequant_fast(float q, float scale, float zero, float col) {
+    const float r = (q * scale + zero) * col;
+    return r == r ? r : dequant_x(q, scale, zero, col);
+}
+
+typedef uint16_t half4_t __attribute__((ext_vector_type(4), aligned(2)));
+
+template <int D>
+__global__ __launch_bounds__(256) void decode_tile_kernel(const sj_kvarn_layout l, const uint8_t * body, float * out_k,
+                                                          float * out_v) {
+    constexpr int NQ = D / 4, WGS = D / 64;      // channel quads; workgroups per record and side
+    __shared__ float cb[512];
+    const int is_v = blockIdx.y, bits = is_v ? l.bits_v : l.bits_k;
+    const bool trellis = l.body == SJKVARN_BODY_TRELLIS, frag = frag_side(l, bits);
+    const size_t r = blockIdx.x / WGS;
+    const int u = (int) (blockIdx.x % WGS) * 256 + (int) threadIdx.x;
+    const int d0 = 4 * (u % NQ), tb = u / NQ >> 1, hf = u / NQ & 1;    // 16-token block, its half
+    const uint8_t * rec = body + r * l.bytes, * pay = rec + (is_v ? l.v_payload : l.k_payload);
+    // this thread's tokens, t0 .. + 3 and t1 .. + 3: in the 4-bit order the halves of a block interleave by fours
+    const int t0 = 16 * tb + (frag ? 4 : 8) * hf, t1 = t0 + (frag ? 8 : 4);
+
+    // everything read is asked for before the codebook's barrier
+    auto halves = [&](uint32_t off) { return *(const half4_t *) (rec + off); };
+    half4_t ts[2], tz[2], ca, cz = {};           // per token: V scale and zero, or the K column scale; per channel
+    ts[0] = halves((is_v ? l.v_scale : l.k_tok) + 2u * (uint32_t) t0);
+    ts[1] = halves((is_v ? l.v_scale : l.k_tok) + 2u * (uint32_t) t1);
+    tz[0] = halves((is_v ? l.v_zero : l.k_tok) + 2u * (uint32_t) t0);
+    tz[1] = halves((is_v ? l.v_zero : l.k_tok) + 2u * (uint32_t) t1);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const uint32_t ci = 2u * (uint32_t) (is_v ? v_ch_idx(l, d0 + c) : k_ch_idx(l, d0 + c));
+        ca[c] = *(const uint16_t *) (rec + (is_v ? l.v_ch : l.k_scale) + ci);
+        if (!is_v) cz[c] = *(const uint16_t *) (rec + l.k_zero + ci);
+    }
+    uint32_t x[8] = {};
+    if (trellis) {
+        // channel d's bits from 6 before its token t0 on (from its start where that lies before it): token t0 + k's
+        // window is the 6 + bits bits ending with its code
+        const int at = t0 ? t0 * bits - 6 : 0, w0 = at >> 5, w1 = w0 + 1 < 4 * bits ? w0 + 1 : w0;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const uint32_t * w = (const uint32_t *) pay + (d0 + c) * 4 * bits;
+            x[c] = __builtin_amdgcn_alignbit(w[w1], w[w0], (uint32_t) at & 31u) << (t0 ? 0 : 6);
+        }
+        const uint16_t * t = codebook(bits, is_v);
+        for (int i = (int) threadIdx.x; i < (64 << bits); i += 256) cb[i] = f16_to_f32(t[i]);
+        __syncthreads();
+    } else if (frag && !is_v) {
+        // 16-token x 16-channel tiles of 32 words, a = token, b = channel: 4 channels in two words
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t * w = (const uint32_t *) pay + (tb * (D / 16) + (d0 >> 4)) * 32 + 4 * (4 * hf + k) + ((d0 >> 1) & 3);
+            x[2 * k] = w[0];
+            x[2 * k + 1] = w[1];
+        }
+    } else if (frag) {
+        // a = channel, b = token: a channel's tokens t0 .. + 3 and t1 .. + 3 in two words
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int d = d0 + c;
+            const uint32_t * w = (const uint32_t *) pay + (tb * (D / 16) + (d >> 4)) * 32 + 4 * (d & 7) + 2 * hf;
+            x[2 * c] = w[0];
+            x[2 * c + 1] = w[1];
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {            // token-major: 4 codes of 2 or 3 bits from bit 0 or 4 of a byte
+            const uint32_t bit = ((uint32_t) ((k < 4 ? t0 : t1 - 4) + k) * D + (uint32_t) d0) * (uint32_t) bits;
+            x[k] = (pay[bit >> 3] | ((bits > 2 ? (uint32_t) pay[(bit >> 3) + 1] : 0u) << 8)) >> (bit & 7u);
+        }
+    }
+
+    // halves by the hardware's conversion: it quiets a NaN and keeps its sign, which is all that dequant_x keeps
+    float a[4], b[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) { a[c] = f16_to_f32_fast(ca[c]); b[c] = f16_to_f32_fast(cz[c]); }
+    float * out = (is_v ? out_v : out_k) + r * 128u * D + d0;
+    auto emit = [&](auto && code) {              // code(k, c): the code's value, token k, channel c
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const float s = f16_to_f32_fast(ts[k >> 2][k & 3]), z = f16_to_f32_fast(tz[k >> 2][k & 3]);
+            float4 y;
+            float * yc = &y.x;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                yc[c] = dequant_fast(code(k, c), is_v ? s : a[c], is_v ? z : b[c], is_v ? a[c] : s);
+            *(float4 *) (out + (size_t) ((k < 4 ? t0 : t1 - 4) + k) * D) = y;
+        }
+    };
+    const uint32_t mask = (1u << bits) - 1u;
+    if (trellis) emit([&](int k, int c) { return cb[(x[c] >> (k * bits)) & ((64u << bits) - 1u)]; });
+    else if (frag && !is_v) emit([&](int k, int c) { return (float) ((x[2 * (k & 3) + (c >> 1)] >> (4 * (k >> 2) + 16 * (c & 1) + (d0 & 8))) & 15u); });
+    else if (frag) emit([&](int k, int c) { return (float) ((x[2 * c + ((k >> 1) & 1)] >> (4 * (((d0 + c) >> 3) & 1) + 16 * (k & 1) + 8 * (k >> 2))) & 15u); });
+    else emit([&](int k, int c) { return (float) ((x[k] >> (c * bits)) & mask); });
+}
+
+// what decode_tile_kernel reads and writes in words: a layer's own geometry, code words at multiples of 4 bytes, halves
+// at even addresses, output rows at multiples of 16
+static bool decode_tiles_ok(const sj_kvarn_layout & l, const void * body, const void * out_k, const void * out_v) {
+    if (!sjk_hip_supported(&l) || (l.body == SJKVARN_BODY_TRELLIS && (l.bits_k > 3 || l.bits_v > 3))) return false;
+    const uint32_t half = l.k_scale | l.k_zero | l.k_tok | l.v_ch | l.v_scale | l.v_zero;
+    const uintptr_t word = (uintptr_t) body | l.bytes | l.k_payload | l.v_payload;
+    return !(word & 3u) && !(half & 1u) && !(((uintptr_t) out_k | (uintptr_t) out_v) & 15u);
+}
+
 // Gather / scatter of device byte runs (the sequence state stream: sink, records and ring rows of every layer
 // to or from one staging buffer). Workgroups stride over the runs; the run descriptor is wave-uniform.
 __global__ __launch_bounds__(256) void copy_runs_kernel(const CopyRun * runs, int n) {
@@ -555,6 +668,12 @@ extern "C" int sjk_hip_decode(const sj_kvarn_layout * l, const uint8_t * d_body,
     if (!l || !d_body || !d_out_k || !d_out_v || n_rec < 0) return SJKVARN_ERR_ARG;
     const size_t n = (size_t) n_rec * l->G * l->D;
     if (!n) return 0;
+    if (decode_tiles_ok(*l, d_body, d_out_k, d_out_v)) {
+        const dim3 grid((unsigned) n_rec * (unsigned) (l->D / 64), 2);
+        if (l->D == 256) hipLaunchKernelGGL(decode_tile_kernel<256>, grid, dim3(256), 0, (hipStream_t) stream, *l, d_body, d_out_k, d_out_v);
+        else hipLaunchKernelGGL(decode_tile_kernel<128>, grid, dim3(256), 0, (hipStream_t) stream, *l, d_body, d_out_k, d_out_v);
+        return SJK_CHECK_LAUNCH();
+    }
     hipLaunchKernelGGL(decode_kernel, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, (hipStream_t) stream, *l, d_body,
                        n_rec, d_out_k, d_out_v);
     return SJK_CHECK_LAUNCH();

@@ -529,3 +529,37 @@ def test_dropin_host_api(oracle, lib):
     lib.sj_kvarn_stage_row(0, cabi.ptr(xa, cabi.f32p), qa.ctypes.data, D)
     oracle.stage_row(0, cabi.ptr(xb, cabi.f32p), qb.ctypes.data, D)
     assert np.array_equal(qa, qb)
+
+
+BODIES = [(bk, bv, 0) for bk in (4, 3, 2) for bv in (4, 3, 2)] + [(3, 3, 1), (3, 2, 1), (2, 2, 1)]
+
+
+@pytest.mark.parametrize("D", [128, 256])
+@pytest.mark.parametrize("bk,bv,body", BODIES, ids=["%d/%d%s" % (a, b, "t" if c else "s") for a, b, c in BODIES])
+def test_decode_word_and_byte_paths(oracle, lib, dev, bk, bv, body, D):
+    """Records of random bytes (every code, every half, subnormals, infinities and NaNs among them), three of them so
+    that the last workgroup ends inside a batch: the word path (aligned records and rows) and the byte path (records
+    at an odd address, rows at a multiple of 4 only) give the same bits, and both are the oracle's rows (a NaN is a
+    NaN: where two NaNs meet the oracle's compiler picks the operand whose sign stays)."""
+    lay = oracle.layout(D, 128, bk, bv, body)
+    n = 3
+    rec = np.random.default_rng(D + 16 * bk + bv + 100 * body).integers(0, 256, n * lay.bytes).astype(np.uint8)
+    size = n * 128 * D * 4
+    rows = []
+    for off in (0, 1):
+        dR = dev.put(np.concatenate([np.zeros(off, np.uint8), rec, np.zeros(4, np.uint8)]))
+        outs = [dev.put(np.full(size // 4 + 4, -7.0, np.float32)) for _ in range(2)]
+        sjk.check(lib.sjk_hip_decode(C.byref(play(lay)), C.c_void_p(dR.value + off), n,
+                                     *(C.c_void_p(o.value + 4 * off) for o in outs), None), "sjk_hip_decode")
+        got = [dev.get(o, size + 16, np.float32) for o in outs]
+        for g in got:
+            assert (g[:off] == -7.0).all() and (g[off + size // 4:] == -7.0).all()     # nothing outside the rows
+        rows.append([np.ascontiguousarray(g[off:off + size // 4]).reshape(n, 128, D) for g in got])
+    row = np.zeros(D, np.float32)
+    for side, fn in enumerate((oracle.decode_k_row, oracle.decode_v_row)):
+        assert np.array_equal(rows[0][side].view(np.uint32), rows[1][side].view(np.uint32))
+        for r in range(n):
+            one = np.ascontiguousarray(rec.reshape(n, -1)[r])
+            for t in range(128):
+                fn(C.byref(lay), cabi.ptr(one), t, cabi.ptr(row, cabi.f32p))
+                assert inputs.floats_equal_nan_unsigned(rows[0][side][r, t], row).all(), (r, t)
