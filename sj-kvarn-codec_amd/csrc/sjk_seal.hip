@@ -394,9 +394,9 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 // p = 2 p + (bit `lane` of m), one instruction. m must come from the scalar unit (a mask straight from a vector
 // compare needs two wait states before a vector instruction reads it, which the compiler does not insert for asm).
 SJK_DEV uint32_t shift_in(uint32_t p, uint64_t m) {
-    uint32_t r;
-    asm("v_addc_co_u32_e64 %0, vcc, %1, %1, %2" : "=v"(r) : "v"(p), "s"(m) : "vcc");
-    return r;
+    // in place: a new register could be one that an MFMA has just used, and asm gets no wait states
+    asm("v_addc_co_u32_e64 %0, vcc, %0, %0, %1" : "+v"(p) : "s"(m) : "vcc");
+    return p;
 }
 
 // lane I of v = x (uniform)
