@@ -41,32 +41,19 @@
 // hi / lo of both codes); fp16 rows are read from HBM where they are used. K values go through
 // v_mfma_f32_16x16x32_f16 (Q hi + lo, K hi + lo for tq6_0), V values through v_mfma_f32_16x16x16_f16,
 // the tq6_0 block norms are applied to the K accumulator and folded into P for V.
-#include "sjk_dev.h"
+#include "sjk_mfma.h"
 
 #include <atomic>
 #include <type_traits>
 
 namespace sjk {
 
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u2 __attribute__((ext_vector_type(2)));
-
 constexpr int A3_NT = 256;
 constexpr int A3_Q = 16;
-constexpr int A3_D = 256;
 constexpr int A3_CH = 16;                        // positions per row chunk
 constexpr int A3_STAGE = A3_CH * 2 * 2 * SJKVARN_TQ6_BLOCK_BYTES;   // LDS bytes per wavefront: 16 tq6_0 K | V rows
 constexpr int A3_PSTRIDE = A3_Q * (A3_D + 2);    // floats per partial
 
-// record layout at head dimension D (256 unless given), G = 128 with BK / BV bits per K / V code
-// (sj_kvarn.h:771-790): K payload | V payload | Kscale[D] | Kzero[D] | Ktok[G] | Vch[D] | Vscale[G] | Vzero[G]
-template <int BK, int BV, int D = A3_D> struct RecLay {
-    static constexpr int VPAY = 16 * D * BK, KSC = VPAY + 16 * D * BV, KZE = KSC + 2 * D, KTOK = KZE + 2 * D,
-                         VCH = KTOK + 256, VSC = VCH + 2 * D, VZE = VSC + 256, BYTES = VZE + 256;
-};
 constexpr int R_VPAY = RecLay<4, 4>::VPAY, R_KSC = RecLay<4, 4>::KSC, R_KZE = RecLay<4, 4>::KZE,
               R_KTOK = RecLay<4, 4>::KTOK, R_VCH = RecLay<4, 4>::VCH, R_VSC = RecLay<4, 4>::VSC,
               R_VZE = RecLay<4, 4>::VZE, R_BYTES = RecLay<4, 4>::BYTES;
@@ -80,27 +67,6 @@ template <int D> struct RecLay4 {
 };
 static_assert(RecLay4<256>::BYTES == R_BYTES && RecLay4<256>::VCH == R_VCH && RecLay4<128>::BYTES == 17920,
               "4/4 record sizes of sj_kvarn.h:792-794 (D = 256, 128)");
-
-// Trellis pair tables: entry e (6 + 2B bits of a channel stream, oldest bit first) holds the fp16
-// codebook values of the two windows it contains, cb[e & (2^(6+B) - 1)] | cb[e >> B] << 16.
-template <int B> struct PairTab { uint32_t v[1 << (6 + 2 * B)]; };
-template <int B, int NC>
-constexpr PairTab<B> make_pairs(const uint16_t (&cb)[NC]) {
-    PairTab<B> t{};
-    for (uint32_t e = 0; e < (1u << (6 + 2 * B)); ++e)
-        t.v[e] = (uint32_t) cb[e & ((1u << (6 + B)) - 1u)] | ((uint32_t) cb[e >> B] << 16);
-    return t;
-}
-constexpr uint16_t k_cb3k[512] = SJK_CB3_K_INIT, k_cb3v[512] = SJK_CB3_V_INIT;
-constexpr uint16_t k_cb2k[256] = SJK_CB2_K_INIT, k_cb2v[256] = SJK_CB2_V_INIT;
-static __device__ const PairTab<3> g_pair3k = make_pairs<3>(k_cb3k);
-static __device__ const PairTab<3> g_pair3v = make_pairs<3>(k_cb3v);
-static __device__ const PairTab<2> g_pair2k = make_pairs<2>(k_cb2k);
-static __device__ const PairTab<2> g_pair2v = make_pairs<2>(k_cb2v);
-template <int B, bool IS_V> SJK_DEV const uint32_t * pair_tab() {
-    if (B == 3) return IS_V ? g_pair3v.v : g_pair3k.v;
-    return IS_V ? g_pair2v.v : g_pair2k.v;
-}
 
 struct A3Args {
     sjk_hip_view v;
@@ -169,24 +135,6 @@ template <typename RL, int NW = 4> struct A3LdsT {
     alignas(16) float wf[NW][A3_Q];              // merge factors exp2(m_w - M) per wave and query
 };
 
-SJK_DEV f4 mfma32(const u4 & a, const u4 & b, const f4 & c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a), __builtin_bit_cast(h8, b), c, 0, 0, 0);
-}
-
-SJK_DEV f4 mfma16(const u2 & a, const u2 & b, const f4 & c) {
-    return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(h4, a), __builtin_bit_cast(h4, b), c, 0, 0, 0);
-}
-
-SJK_DEV float h2f(uint32_t bits16) { return (float) __builtin_bit_cast(_Float16, (uint16_t) bits16); }
-
-// (x0, x1) as fp16 pairs {hi, lo}: hi = RN16(x), lo = RN16(x - hi)
-SJK_DEV u2 split2(float x0, float x1) {
-    const _Float16 a = (_Float16) x0, b = (_Float16) x1;
-    const _Float16 c = (_Float16) (x0 - (float) a), d = (_Float16) (x1 - (float) b);
-    return u2{(uint32_t) __builtin_bit_cast(uint16_t, a) | ((uint32_t) __builtin_bit_cast(uint16_t, b) << 16),
-              (uint32_t) __builtin_bit_cast(uint16_t, c) | ((uint32_t) __builtin_bit_cast(uint16_t, d) << 16)};
-}
-
 // v_fma_mix: fp32 a times the low / high fp16 half of h2 (plus fp32 c), the exact product rounded once, to
 // fp32. Inline asm: never pass these a register written by an MFMA (no hazard wait states are inserted for
 // asm operands).
@@ -200,9 +148,6 @@ SJK_DEV float mul_hi(float a, uint32_t h2) {
     asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(r) : "v"(a), "v"(h2));
     return r;
 }
-SJK_DEV float fma_lo(float a, uint32_t h2, float c) { return __builtin_fmaf(a, h2f(h2 & 0xFFFFu), c); }
-SJK_DEV float fma_hi(float a, uint32_t h2, float c) { return __builtin_fmaf(a, h2f(h2 >> 16), c); }
-
 // fp16 pair {RN16(a0 * s.lo), RN16(a1 * s.hi)}: v_fma_mixlo / mixhi round the exact product once and write
 // one half of the destination, keeping the other (the mixlo result's high half is whatever the register
 // held, until the mixhi writes it). The compiler inserts no hazard wait states around inline asm (it does not
@@ -230,30 +175,6 @@ SJK_DEV u2 mul_split(float a0, float a1, uint32_t s) {
     return u2{hi, lo};
 }
 
-// Row exchange between two registers: v_permlane16_swap_b32 swaps the odd 16-lane rows of x with the even
-// rows of y, v_permlane32_swap_b32 the upper 32 lanes of x with the lower 32 of y (no LDS round trip, unlike
-// a lane shuffle). Written out as asm because this toolchain's builtin returns the first register for both
-// results; s_nop 1 gives the wait states a VALU write needs before the swap reads it. Never pass an MFMA result.
-SJK_DEV void swap16(uint32_t & x, uint32_t & y) { asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(x), "+v"(y)); }
-SJK_DEV void swap32(uint32_t & x, uint32_t & y) { asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(x), "+v"(y)); }
-
-// sum / max over the four 16-lane rows of a wavefront (the MFMA lane groups g), (r0 + r1) + (r2 + r3), the
-// same value in every lane
-SJK_DEV float rows_sum(float v) {
-    uint32_t a = __builtin_bit_cast(uint32_t, v), b = a;
-    swap16(a, b);
-    uint32_t c = __builtin_bit_cast(uint32_t, __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b)), d = c;
-    swap32(c, d);
-    return __builtin_bit_cast(float, c) + __builtin_bit_cast(float, d);
-}
-SJK_DEV float rows_max(float v) {
-    uint32_t a = __builtin_bit_cast(uint32_t, v), b = a;
-    swap16(a, b);
-    uint32_t c = __builtin_bit_cast(uint32_t, fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b))), d = c;
-    swap32(c, d);
-    return fmaxf(__builtin_bit_cast(float, c), __builtin_bit_cast(float, d));
-}
-
 // max / sum over all 64 lanes: DPP rotations inside the rows, then across the rows (same value in every lane)
 SJK_DEV float wave_max(float v) {
     v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xF, 0xF, false)));
@@ -270,31 +191,6 @@ SJK_DEV float wave_sum(float v) {
     return rows_sum(v);
 }
 
-// unsigned max over all 64 lanes: DPP rotations inside the rows, then across the rows
-SJK_DEV uint32_t wave_umax(uint32_t v) {
-    v = max(v, (uint32_t) __builtin_amdgcn_update_dpp(0, (int) v, 0x128, 0xF, 0xF, false));    // row_ror:8
-    v = max(v, (uint32_t) __builtin_amdgcn_update_dpp(0, (int) v, 0x124, 0xF, 0xF, false));    // row_ror:4
-    v = max(v, (uint32_t) __builtin_amdgcn_update_dpp(0, (int) v, 0x122, 0xF, 0xF, false));    // row_ror:2
-    v = max(v, (uint32_t) __builtin_amdgcn_update_dpp(0, (int) v, 0x121, 0xF, 0xF, false));    // row_ror:1
-    uint32_t a = v, b = v;
-    swap16(a, b);
-    uint32_t c = max(a, b), d = c;
-    swap32(c, d);
-    return max(c, d);
-}
-
-// Power of two 2^k for the P' operands of one record: with vmax = max_t Vscale[t] in [2^(e-1), 2^e),
-// P' = P * Vscale * 2^k (P <= 1, k = 14 - e) stays below 2^14 and the small weights stay clear of the
-// fp16 subnormal range, where they would lose their low bits. Returns 2^k (uniform over
-// the wave) and inv = 2^-k, by which the product is scaled back. vsc: the record's Vscale[128] in LDS.
-SJK_DEV float pv_scale(const uint8_t * vsc, int lane, float & inv) {
-    const uint32_t wv = *(const uint32_t *) (vsc + 4 * lane);       // Vscale of tokens 2 lane, 2 lane + 1 (>= 0)
-    const uint32_t mx = wave_umax(max(wv & 0xFFFFu, wv >> 16));       // non-negative halves order like their bits
-    const int e = __builtin_amdgcn_frexp_expf(h2f(mx));
-    inv = __builtin_amdgcn_ldexpf(1.0f, e - 14);
-    return __builtin_amdgcn_ldexpf(1.0f, 14 - e);
-}
-
 // Issue priority from a wavefront's progress through its own work (first quarter 3, ..., last quarter 0).
 // Wavefronts that share a SIMD are not issued evenly at equal priority: one finishes well before the other,
 // which then runs alone at a lower rate (the loop ends of the 8 record wavefronts of a CU spread by ~6 us).
@@ -305,12 +201,6 @@ SJK_DEV void prio_by_progress(int done, int total) {
     else if (q == 1) __builtin_amdgcn_s_setprio(2);
     else if (q == 2) __builtin_amdgcn_s_setprio(1);
     else __builtin_amdgcn_s_setprio(0);
-}
-
-SJK_DEV void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // query row n of the tile for KV head h: (position index, global head); rows past n_rows are dead (masked)
@@ -2502,6 +2392,17 @@ extern "C" int sjk_attend3_batch(const sjk_hip_attend_job * jobs, int n_jobs, in
                                  void * stream) {
     const int body = a3_body(jobs[0].v.lay), H = jobs[0].v.n_head_kv;
     const int rows = n_q * (n_head / H);
+    bool wide = true;
+    for (int j = 0; wide && j < n_jobs; ++j)
+        wide = sjk_prefill_takes(jobs[j].v, body, n_q, n_head, jobs[j].d_q, jobs[j].d_out);
+    if (wide) {
+        for (int j = 0; j < n_jobs; ++j) {
+            const sjk_hip_attend_job & J = jobs[j];
+            const int rc = sjk_prefill(J.v, nullptr, 0, J.B, J.N, J.qpos0, n_q, n_head, J.d_q, scale, J.d_out, (hipStream_t) stream);
+            if (rc) return rc;
+        }
+        return 0;
+    }
     A3Batch bt = {};
     for (int j = 0; j < n_jobs; ++j) {
         const sjk_hip_attend_job & J = jobs[j];
@@ -2689,6 +2590,8 @@ extern "C" int sjk_hip_attend_dyn(const sjk_hip_view * v, const int32_t * d_desc
     const int slots = body == 44 ? (cus / H > 0 ? cus / H : 1) : a3_slots(H);
     const int rows = n_q * (n_head / H);
     hipStream_t st = (hipStream_t) stream;
+    if (sjk_prefill_takes(*v, body, n_q, n_head, d_q, d_out))
+        return sjk_prefill(*v, d_desc, n_max, 0, 0, 0, n_q, n_head, d_q, scale, d_out, st);
     A3Batch * plan = (A3Batch *) ws_plan(*v);
     for (int r0 = 0; r0 < rows; r0 += A3_Q * A3_MAXJ) {
         const int lrows = rows - r0 < A3_Q * A3_MAXJ ? rows - r0 : A3_Q * A3_MAXJ, nt = (lrows + A3_Q - 1) / A3_Q;

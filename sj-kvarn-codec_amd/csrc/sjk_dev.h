@@ -224,6 +224,11 @@ int ws_slots(int n_head_kv);
 // compute units of the current device
 int n_cus();
 
+// attention of a call with many query rows per KV head (sjk_prefill.hip); desc and n_max: sjk_hip_attend_dyn
+int sjk_prefill(const sjk_hip_view & v, const int32_t * desc, uint32_t n_max, uint32_t B, uint32_t N, uint32_t qpos0,
+                int n_q, int n_head, const float * d_q, float scale, float * d_out, hipStream_t st);
+// whether that kernel takes the call: the body, the number of query rows, the buffers
+bool sjk_prefill_takes(const sjk_hip_view & v, int body, int n_q, int n_head, const float * d_q, const float * d_out);
 }  // namespace sjk
 
 #define SJK_CHECK_LAUNCH() (hipPeekAtLastError() == hipSuccess ? 0 : SJK_ERR_DEVICE)

@@ -304,3 +304,70 @@ def test_wide_rows_vs_oracle(oracle, lib, dev, D, H, bk, bv, body, n_q, n_head, 
     finally:
         oracle.layer_free(C.byref(OL))
         lib.sj_kvarn_layer_free(C.byref(PL))
+
+
+PREFILL = [
+    # D, H, gq, n_q, staging, sink_type, sealed groups, tail, first query position before the end, scale
+    (256, 4, 4, 64, 0, 0, 9, 301, 64, 0.0625),     # 256 rows, the fewest; a tail that is no multiple of 32
+    (128, 4, 4, 67, 0, 0, 9, 256, 67, 0.08),       # a last tile of 12 rows
+    (256, 1, 16, 17, 0, 0, 0, 0, 128, 0.0625),     # causal in a sink that is all there is
+    (256, 2, 8, 33, 0, 1, 3, 470, 300, 0.0625),    # sink in the staging type, rows across the body's end
+    (128, 2, 4, 100, 1, 0, 4, 290, 600, -0.05),    # fp16 staging, a negative scale, later records masked
+    (256, 4, 4, 64, 1, 1, 2, 257, 64, 0.0),        # fp16 sink in the staging type, scale 0 (plain means)
+    (128, 16, 4, 65, 0, 0, 1, 260, 65, 0.08),      # more tiles than there are compute units
+]
+
+
+@pytest.mark.parametrize("D,H,gq,n_q,staging,sink_type,ngr,tail,back,scale", PREFILL)
+def test_prefill_kernel_edges(oracle, lib, dev, D, H, gq, n_q, staging, sink_type, ngr, tail, back, scale):
+    """Calls of 256 query rows per KV head and more: ragged tiles, every region and staging type, causal rows in each
+    region, each against the oracle; the descriptor call gives the same bits, and a call whose output lies over its
+    queries (which takes the 16-row kernels) agrees with the oracle too."""
+    S, G = 128, 128
+    B = S + ngr * G
+    n_pos = B + tail
+    OL, PL = make_pair(oracle, lib, D, H, 4, 4, 0, 256, 512, n_ctx=4096, n_ubatch=512, staging=staging, sink_type=sink_type)
+    view = lib.sjk_layer_view(C.byref(PL))
+    try:
+        K, V = inputs.kv_rows(n_pos, H, D, seed=70 + D + ngr)
+        dK, dV = dev.put(K), dev.put(V)
+        done = S
+        for p in range(0, n_pos, 256):             # the ring holds no more at once
+            n = min(256, n_pos - p)
+            view_at = lambda d, off: C.c_void_p(d.value + 4 * off * H * D)
+            sjk.check(lib.sjk_hip_layer_store(C.byref(view), p, n, view_at(dK, p), view_at(dV, p), 1, None), "layer_store")
+            full = min(B, S + (p + n - S) // G * G) if p + n > S else S
+            if full > done:
+                sjk.check(lib.sjk_hip_commit(C.byref(view), 1, done, full, 16, None), "commit")
+                done = full
+        assert done == B
+        dev.sync()
+        sink_b = S * H * (4 * D if sink_type == 0 else 2 * OL.stage_bytes)
+        for name, nb in (("sink", sink_b), ("ring", OL.cap * H * 2 * OL.stage_bytes), ("body", ngr * H * OL.lay.bytes)):
+            if nb:
+                b = dev.get(C.c_void_p(getattr(view, name)), nb, np.uint8)
+                C.memmove(getattr(OL, name), b.ctypes.data, nb)
+        n_head, qpos0 = H * gq, max(0, n_pos - back)
+        q = np.random.default_rng(3 + n_q).standard_normal((n_q, n_head, D)).astype(np.float32)
+        q[0] *= 1e-6                               # a row's scale is its own
+        got = attend(lib, dev, view, B, n_pos, qpos0, q, scale)
+        rng = np.random.default_rng(n_q)
+        rows = sorted({(0, 0), (1, n_head - 1), (n_q - 1, 0), (n_q - 1, n_head - 1)} |
+                      {(int(a), int(b)) for a, b in zip(rng.integers(0, n_q, 60), rng.integers(0, n_head, 60))})
+        want = oracle_rows(oracle, OL, B, n_pos, q, qpos0, scale, rows)
+        worst, l2 = check_rows(got, want)
+        desc = np.zeros(16, np.int32)
+        desc[2], desc[3], desc[4] = B, n_pos, qpos0
+        dq, do, dd = dev.put(q), dev.put(q), dev.put(desc)
+        sjk.check(lib.sjk_hip_attend(C.byref(view), B, n_pos, qpos0, n_q, n_head, do, scale, do, None), "attend over q")
+        check_rows(dev.get(do, q.nbytes, np.float32).reshape(q.shape), want)
+        sjk.check(lib.sjk_hip_attend_dyn(C.byref(view), dd, 4096, n_q, n_head, dq, scale, do, None), "attend_dyn")
+        assert np.array_equal(dev.get(do, q.nbytes, np.uint32), got.reshape(-1).view(np.uint32))
+        desc[2] = 4095                             # no whole number of groups: NaN rows
+        bad = dev.put(desc)
+        sjk.check(lib.sjk_hip_attend_dyn(C.byref(view), bad, 4096, n_q, n_head, dq, scale, do, None), "attend_dyn")
+        assert np.isnan(dev.get(do, q.nbytes, np.float32)).all()
+        say("[tiles] prefill D=%d %d rows: worst %.4f of the tolerance, rel L2 %.2e" % (D, n_q * gq, worst, l2))
+    finally:
+        oracle.layer_free(C.byref(OL))
+        lib.sj_kvarn_layer_free(C.byref(PL))

@@ -201,3 +201,16 @@ def test_seal_kernel_uses_no_scratch():
     assert len(kernels) == 2, sorted(res)           # D = 128 and D = 256
     for k in kernels:
         assert res[k].get("ScratchSize [bytes/lane]", -1) == 0, (k, res[k])
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc is not installed")
+def test_prefill_kernel_has_no_scratch_and_keeps_its_wait_states():
+    # a spill of its 128 O registers costs more than the kernel itself
+    res = resources("sjk_prefill.hip")
+    kernels = [k for k in res if "prefill_kernel" in k]
+    assert len(kernels) >= 2, sorted(res)
+    for k in kernels:
+        assert res[k].get("ScratchSize [bytes/lane]", -1) == 0, (k, res[k])
+    _, asm = compile_device("sjk_prefill.hip")
+    for k, lines in kernel_bodies(asm).items():
+        assert not asm_mfma_hazards(lines), k
