@@ -343,7 +343,8 @@ int sjk_hip_commit_dyn(const sjk_hip_view * views, int n_layers, const int32_t *
  * (sj_kvarn_cuda.cuh:102-135). d_q, d_out: [n_q][n_head][D] fp32, rotated basis; GQA maps query head
  * hq to KV head hq / (n_head / n_head_kv). Any n_q and n_head (a prefill ubatch as well as a decode step):
  * the n_q x n_head / n_head_kv query rows of a KV head are cut into tiles of 16 rows, and a launch takes up to
- * 8 jobs side by side (sharing its workgroups in proportion to their work; each job reads the context). The
+ * 8 jobs side by side (sharing its workgroups in proportion to their work; each job reads the context); a 4/4
+ * call of 256 rows and more whose output does not lie over its queries runs in one launch of 32-row tiles. The
  * partial results go to v->work (SJKVARN_ERR_ARG without one). Every layout a layer can have runs
  * on a matrix-core kernel; a hand-built view outside them (another group size, head dimension or record
  * layout) is refused with SJK_ERR_UNSUPPORTED and a message (sjk_last_error), as are the batched, no-alloc and
@@ -372,8 +373,8 @@ int sjk_hip_attend_noalloc(const sjk_hip_view * v, uint32_t B, uint32_t N, uint3
  * plan kernel that writes the launch's job table into v->work. The table and the partial results live in v->work,
  * which the layer allocated when it was created, so a capture sees no allocation. Any number of query rows per
  * KV head (n_q x n_head / n_head_kv): as in sjk_hip_attend, 16-row tiles, up to 8 a launch, shared out by the
- * same arithmetic; a launch and its combine per 8 tiles, in stream order, all on the one stream a capture
- * records. */
+ * same arithmetic, a launch and its combine per 8 tiles, or the 32-row tiles of a large 4/4 call, with no plan
+ * kernel; in stream order, all on the one stream a capture records. */
 int sjk_hip_attend_dyn(const sjk_hip_view * v, const int32_t * d_desc, uint32_t n_max, int n_q, int n_head,
                        const float * d_q, float scale, float * d_out, void * stream);
 

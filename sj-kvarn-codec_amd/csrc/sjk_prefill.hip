@@ -22,7 +22,7 @@
 // What bounds it (D = 256): vector issue. A record is 128 + 64 products of 32 cycles, 6,100 cycles of a SIMD's matrix
 // core, and about 2,300 vector instructions, 10,000 cycles at their measured 2.5-5 each; 32 staged positions 96
 // products and 1,900 instructions. Two wavefronts per SIMD (O alone is 128 of their 256 registers) overlap the two only in
-// part. 512 positions x 16 heads at 32K, D = 256: 672 us against 1,322 us with the 16-row kernels (5.5K staged
+// part. 512 positions x 16 heads at 32K, D = 256: 660 us against 1,322 us with the 16-row kernels (5.5K staged
 // positions; 275 GFLOP of products at one pass, 0.41 PFLOP/s).
 #include "sjk_mfma.h"
 
@@ -37,7 +37,7 @@ constexpr int PF_CH = 32;                        // staged positions per step
 constexpr int PF_MSTR = 68;                      // floats per query row of a merge slice (64 channels, 16-byte rows)
 constexpr int PF_WAVE = PF_ROWS * PF_MSTR * 4;   // LDS bytes per wavefront
 
-// cost of 32 staged positions and of a sealed record: 3 : 4 took 672 us, 7 : 10 688 us, 2 : 3 682 us and 5 : 9 725 us on
+// cost of 32 staged positions and of a sealed record: 3 : 4 was the fastest; 7 : 10 took 2% longer, 2 : 3 1.5% and 5 : 9 8% on
 // the 32K ubatch above
 constexpr int PF_COST_CH = 3, PF_COST_REC = 4;
 
