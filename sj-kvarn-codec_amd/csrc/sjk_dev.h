@@ -56,6 +56,13 @@ SJK_DEV float f16_to_f32(uint16_t h) {
 // NaNs; used where only values matter (attention), never for bytes that are compared
 SJK_DEV float f16_to_f32_fast(uint16_t h) { return (float) __builtin_bit_cast(_Float16, h); }
 
+// LDS written by lanes of this wavefront is read by others of it
+SJK_DEV void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---- the host's NaN rule, for the paths that see non-finite values ----
 // A stored NaN half keeps only its sign (sign | 0x7E00), so the sign of every NaN the arithmetic makes is part
 // of the bytes. IEEE 754 leaves it unspecified; the reference's host build (x86-64 SSE) returns a quieted copy of

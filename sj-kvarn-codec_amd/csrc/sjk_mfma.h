@@ -110,10 +110,4 @@ SJK_DEV float pv_scale(const uint8_t * vsc, int lane, float & inv) {
     return __builtin_amdgcn_ldexpf(1.0f, 14 - e);
 }
 
-SJK_DEV void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 }  // namespace sjk

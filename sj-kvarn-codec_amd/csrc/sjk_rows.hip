@@ -7,13 +7,21 @@
 //     1/sqrt(D). Same stage order and operations as the reference, so bit-identical.
 //   * tq6_0 (sj_kvarn.h:1221-1247): the two per-block sums (x^2, then centroid^2) must be sequential
 //     fp32 sums over the 128 values in index order. The squares are formed in parallel, written to
-//     LDS, and every lane of the block walks them in order with broadcast reads, so each lane ends
-//     with the block's exact sum. The level search, packing and stores are parallel over lanes.
+//     LDS and walked in order: in a small call by every lane of the block with broadcast reads, in a
+//     large one by one lane per block, the workgroup's blocks side by side in one wavefront. The level
+//     search, packing and stores are parallel over lanes.
 #include "sjk_dev.h"
 
 namespace sjk {
 
-constexpr int ROW_WAVES = 4;                 // wavefronts (rows) per workgroup
+// Wavefronts (rows) per workgroup. A walk takes 32 16-byte LDS reads whatever the number of lanes that use it, so
+// with a walk per row (ROW_WAVES) a large tq6_0 call is bound by them; with the walks of a workgroup's rows in one
+// wavefront's lanes (ROW_WAVES_BIG) the others wait at a barrier, which costs a small call its latency. Appends at
+// D = 128 / 256, walk per row against one wavefront's: 2,048 rows 4.7 / 5.2 against 5.8 / 6.8 us, 4,096 rows 6.1 / 7.0
+// against 6.0 / 6.9, 8,192 rows 8.7 / 10.7 against 7.5 / 9.1: the line is at a large workgroup per CU. Rows that are no
+// tq6_0 leave before the walks; among them the small workgroups are the faster at every size (8,192 fp16 rows 4.4 /
+// 5.1 against 5.1 / 6.0 us, with the walks 9.0 / 11.0).
+constexpr int ROW_WAVES = 4, ROW_WAVES_BIG = 16;
 enum { OUT_F32 = 0, OUT_F16 = 1, OUT_TQ6 = 2 };
 
 struct RowJob {
@@ -96,17 +104,40 @@ SJK_DEV void hadamard_row(float (&x)[V], int lane, float scale) {
     for (int m = 0; m < V; ++m) x[m] = XN ? xmul(x[m], scale) : x[m] * scale;
 }
 
-template <int V>
-__global__ __launch_bounds__(64 * ROW_WAVES) void rows_kernel(const RowBatch bt) {
-    constexpr int D = 64 * V;
-    __shared__ float s_sq[ROW_WAVES][D];
-    __shared__ float s_mid[64], s_cent[64];
+// the sum of 128 values in index order; XN: the host's NaN rule
+template <bool XN> SJK_DEV float walk(const float * sq) {
+    const float4 * p = (const float4 *) sq;
+    float s = 0.0f;
+    if (XN) {
+        for (int i = 0; i < 32; ++i) {
+            const float4 q = p[i];
+            s = xadd(s, q.x); s = xadd(s, q.y); s = xadd(s, q.z); s = xadd(s, q.w);
+        }
+    } else {
+#pragma unroll 8
+        for (int i = 0; i < 32; ++i) {
+            const float4 q = p[i];
+            s = s + q.x; s = s + q.y; s = s + q.z; s = s + q.w;
+        }
+    }
+    return s;
+}
+
+template <int V, int NW>
+__global__ __launch_bounds__(64 * NW) void rows_kernel(const RowBatch bt) {
+    constexpr bool BIG = NW > ROW_WAVES;   // one wavefront walks the blocks of all rows
+    constexpr int NB = V / 2;              // 128-value blocks of a row
+    constexpr int BS = 132;                // floats from block to block: the walking lanes' reads are in different banks
+    static_assert(NW * NB <= 64, "a lane per block");
+    __shared__ alignas(16) float s_sq[NW * NB * BS];
+    __shared__ float s_mid[64], s_cent[64], s_sum[BIG ? NW * NB : 1];
+    __shared__ bool s_xn[BIG ? NW : 1];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (threadIdx.x < 64) {
         s_mid[threadIdx.x] = threadIdx.x < 63 ? tq6_mid(threadIdx.x) : __builtin_inff();
         s_cent[threadIdx.x] = tq6_cent(threadIdx.x);
     }
-    const int rg = blockIdx.x * ROW_WAVES + wave;             // wave-uniform
+    const int rg = blockIdx.x * NW + wave;                    // wave-uniform
     int ji = 0;
     for (int k = 1; k < bt.n_jobs; ++k) ji += rg >= bt.row_base[k] ? 1 : 0;
     ji = __builtin_amdgcn_readfirstlane(ji);
@@ -133,7 +164,10 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void rows_kernel(const RowBatch bt)
         if (xn) hadamard_row<V, true>(x, lane, j.rot_scale);
         else hadamard_row<V, false>(x, lane, j.rot_scale);
     }
-    __syncthreads();
+    const bool tq = live && mode == OUT_TQ6;
+    bool any_tq = tq;
+    if (BIG) any_tq = __syncthreads_or(tq) != 0;
+    else __syncthreads();
     if (live && mode == OUT_F32) {
         float * o = (float *) dst;
 #pragma unroll
@@ -144,28 +178,29 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void rows_kernel(const RowBatch bt)
 #pragma unroll
         for (int m = 0; m < V; ++m) o[V * lane + m] = f32_to_f16(x[m]);
     }
-    // tq6_0: every wave takes part in the barriers; only tq6 rows use the results
+    if (!any_tq) return;                   // a small call's row, or a workgroup without a tq6_0 row
+    // tq6_0: every wave of a large call's workgroup takes part in the barriers; only tq6 rows use the results
     constexpr int LPB = 128 / V;           // lanes per 128-value block
     const int b = lane / LPB;              // block of this lane
-    float * sq = s_sq[wave];
+    float * blk_sq = s_sq + (wave * NB + b) * BS, * sq = blk_sq + V * (lane % LPB);
+    auto sync = [] {
+        if (BIG) __syncthreads();
+        else wave_sync();
+    };
+    if (BIG && lane == 0) s_xn[wave] = xn;
 #pragma unroll
-    for (int m = 0; m < V; ++m) sq[V * lane + m] = xn ? xmul(x[m], x[m]) : x[m] * x[m];
-    __syncthreads();
-    float nsq = 0.0f;
-    {
-        const float4 * p = (const float4 *) (sq + 128 * b);
-        if (xn) {
-            for (int i = 0; i < 32; ++i) {
-                const float4 q = p[i];
-                nsq = xadd(nsq, q.x); nsq = xadd(nsq, q.y); nsq = xadd(nsq, q.z); nsq = xadd(nsq, q.w);
-            }
-        } else {
-#pragma unroll 8
-            for (int i = 0; i < 32; ++i) {
-                const float4 q = p[i];
-                nsq = nsq + q.x; nsq = nsq + q.y; nsq = nsq + q.z; nsq = nsq + q.w;
-            }
+    for (int m = 0; m < V; ++m) sq[m] = xn ? xmul(x[m], x[m]) : x[m] * x[m];
+    sync();
+    float nsq;
+    if (BIG) {
+        if (threadIdx.x < NW * NB) {
+            const float * p = s_sq + (int) threadIdx.x * BS;
+            s_sum[threadIdx.x] = s_xn[threadIdx.x / NB] ? walk<true>(p) : walk<false>(p);
         }
+        __syncthreads();
+        nsq = s_sum[wave * NB + b];
+    } else {
+        nsq = xn ? walk<true>(blk_sq) : walk<false>(blk_sq);
     }
     const float norm = nsq != nsq ? nan_of(nsq) : __builtin_sqrtf(nsq);
     const bool big = norm > 1e-10f;
@@ -173,21 +208,23 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void rows_kernel(const RowBatch bt)
     int code[V];
 #pragma unroll
     for (int m = 0; m < V; ++m) code[m] = tq6_level(big ? x[m] * inv : 0.0f, s_mid);
-    __syncthreads();
+    if (!BIG) wave_sync();                 // (the barrier after the large call's walk)
 #pragma unroll
-    for (int m = 0; m < V; ++m) { const float c = s_cent[code[m]]; sq[V * lane + m] = c * c; }
-    __syncthreads();
-    float rsq = 0.0f;
-    {
-        const float4 * p = (const float4 *) (sq + 128 * b);
-#pragma unroll 8
-        for (int i = 0; i < 32; ++i) {
-            const float4 q = p[i];
-            rsq = rsq + q.x; rsq = rsq + q.y; rsq = rsq + q.z; rsq = rsq + q.w;
+    for (int m = 0; m < V; ++m) { const float c = s_cent[code[m]]; sq[m] = c * c; }
+    sync();
+    float rsq;
+    if (BIG) {
+        if (threadIdx.x < NW * NB) {
+            const float s = walk<false>(s_sq + (int) threadIdx.x * BS);
+            s_sum[threadIdx.x] = s;        // nsq was read before the last barrier
         }
+        __syncthreads();
+        rsq = s_sum[wave * NB + b];
+    } else {
+        rsq = walk<false>(blk_sq);
     }
     const float rn = __builtin_sqrtf(rsq);
-    if (!(live && mode == OUT_TQ6)) return;
+    if (!tq) return;
     uint8_t * blk = dst + (size_t) b * SJKVARN_TQ6_BLOCK_BYTES;
     const int i0 = V * (lane % LPB);       // index of this lane's first value inside its block
     if (lane % LPB == 0) *(uint16_t *) blk = f32_to_f16(rn > 1e-10f ? xdiv(norm, rn) : norm);
@@ -218,13 +255,21 @@ static int launch_batch(RowBatch & bt, hipStream_t st) {
     for (int k = 0; k < bt.n_jobs; ++k) bt.row_base[k + 1] = bt.row_base[k] + (bt.job[k].n_rows > 0 ? bt.job[k].n_rows : 0);
     const int n_rows = bt.row_base[bt.n_jobs];
     if (n_rows <= 0) return 0;
-    const dim3 grid((unsigned) ((n_rows + ROW_WAVES - 1) / ROW_WAVES)), block(64 * ROW_WAVES);
+    bool tq = false;
+    for (int k = 0; k < bt.n_jobs; ++k)
+        tq |= bt.job[k].kind == 0 ? bt.job[k].out_mode == OUT_TQ6 : bt.job[k].staging != SJKVARN_STAGING_F16;
+    const int nw = tq && n_rows >= ROW_WAVES_BIG * n_cus() ? ROW_WAVES_BIG : ROW_WAVES;
+    const dim3 grid((unsigned) ((n_rows + nw - 1) / nw)), block((unsigned) (64 * nw));
+#define SJK_ROWS(V) \
+    if (nw == ROW_WAVES) hipLaunchKernelGGL((rows_kernel<V, ROW_WAVES>), grid, block, 0, st, bt); \
+    else hipLaunchKernelGGL((rows_kernel<V, ROW_WAVES_BIG>), grid, block, 0, st, bt);
     switch (bt.job[0].D) {
-    case 128: hipLaunchKernelGGL(rows_kernel<2>, grid, block, 0, st, bt); break;
-    case 256: hipLaunchKernelGGL(rows_kernel<4>, grid, block, 0, st, bt); break;
-    case 512: hipLaunchKernelGGL(rows_kernel<8>, grid, block, 0, st, bt); break;
+    case 128: SJK_ROWS(2) break;
+    case 256: SJK_ROWS(4) break;
+    case 512: SJK_ROWS(8) break;
     default: return SJK_ERR_UNSUPPORTED;
     }
+#undef SJK_ROWS
     return SJK_CHECK_LAUNCH();
 }
 

@@ -563,3 +563,59 @@ def test_decode_word_and_byte_paths(oracle, lib, dev, bk, bv, body, D):
             for t in range(128):
                 fn(C.byref(lay), cabi.ptr(one), t, cabi.ptr(row, cabi.f32p))
                 assert inputs.floats_equal_nan_unsigned(rows[0][side][r, t], row).all(), (r, t)
+
+
+@pytest.mark.parametrize("n", [4095, 4096, 4109])
+@pytest.mark.parametrize("D", [128, 256, 512])
+def test_large_row_calls(oracle, lib, dev, D, n):
+    """Calls around the row count from which one wavefront walks the blocks of 16 rows, the last workgroup whole or
+    not: tq6_0 bytes are the oracle's (48 rows hold infinities and NaNs, between finite rows of the same workgroups),
+    rotation and fp16 rows those of smaller calls."""
+    rng = np.random.default_rng(D + n)
+    x = rng.standard_normal((n, D)).astype(np.float32)
+    x[5] = 0.0
+    x[rng.permutation(n)[:48]] = inputs.nonfinite_rows(48, D, seed=n)
+    rb = D // 128 * 98
+    want = np.zeros((n, rb), np.uint8)
+    for r in range(n):
+        row = np.ascontiguousarray(x[r])
+        oracle.tq6_quantize_row(cabi.ptr(row, cabi.f32p), want[r].ctypes.data, D)
+    dx, dq = dev.put(x), dev.put(np.full(n * rb + 64, 77, np.uint8))
+    sjk.check(lib.sjk_hip_stage(0, dx, dq, D, rb, n, None), "sjk_hip_stage")
+    got = dev.get(dq, n * rb + 64, np.uint8)
+    assert (got[n * rb:] == 77).all()
+    assert inputs.tq6_mismatch(got[:n * rb].reshape(n, rb), want).size == 0
+    outs = []
+    for step in (n, 1000):
+        dr, d16 = dev.put(x), dev.alloc(n * D * 2)
+        for i in range(0, n, step):
+            m = min(step, n - i)
+            sjk.check(lib.sjk_hip_rotate(C.c_void_p(dr.value + 4 * D * i), m, D, None), "sjk_hip_rotate")
+            sjk.check(lib.sjk_hip_stage(1, C.c_void_p(dx.value + 4 * D * i), C.c_void_p(d16.value + 2 * D * i), D, 2 * D, m, None), "stage")
+        outs.append((dev.get(dr, n * D * 4, np.uint8), dev.get(d16, n * D * 2, np.uint8)))
+    assert all(np.array_equal(a, b) for a, b in zip(*outs))
+
+
+@pytest.mark.parametrize("sink_type,staging", [(0, 0), (1, 0), (0, 1)])
+@pytest.mark.parametrize("D,H,n_pos", [(256, 4, 513), (128, 8, 267)])
+def test_large_append_across_the_sink(oracle, lib, dev, D, H, n_pos, sink_type, staging):
+    """An append of more than 4096 rows whose positions cross the sink's end (fp16 and tq6_0 rows in one workgroup)
+    writes the bytes of the same append in small pieces."""
+    kv = inputs.kv_rows(n_pos, H, D, seed=D + staging)
+    dk, dv = dev.put(kv[0]), dev.put(kv[1])
+    sb = 2 * D if staging else D // 128 * 98
+    sink_b, ring_b = 128 * H * 4 * D, 640 * H * 2 * sb
+    got = []
+    for step in (n_pos, 31):
+        sink, ring = dev.put(np.zeros(sink_b, np.uint8)), dev.put(np.zeros(ring_b, np.uint8))
+        v = sjk.View()
+        v.lay, v.n_head_kv, v.staging, v.sink_type, v.S, v.cap = sjk.layout(D, 128, 4, 4, 0), H, staging, sink_type, 128, 640
+        v.stage_bytes = sb
+        v.sink, v.ring, v.body = sink.value, ring.value, ring.value
+        for p in range(0, n_pos, step):
+            off = 4 * p * H * D
+            sjk.check(lib.sjk_hip_layer_store(C.byref(v), 101 + p, min(step, n_pos - p), C.c_void_p(dk.value + off),
+                                              C.c_void_p(dv.value + off), 1, None), "layer_store")
+        got.append((dev.get(sink, sink_b, np.uint8), dev.get(ring, ring_b, np.uint8)))
+    assert got[0][0].any() and got[0][1].any()
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
