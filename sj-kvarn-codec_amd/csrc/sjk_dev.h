@@ -63,6 +63,13 @@ SJK_DEV void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Row exchange between two registers: v_permlane16_swap_b32 swaps the odd 16-lane rows of x with the even
+// rows of y, v_permlane32_swap_b32 the upper 32 lanes of x with the lower 32 of y (no LDS round trip, unlike
+// a lane shuffle). Written out as asm because this toolchain's builtin returns the first register for both
+// results; s_nop 1 gives the wait states a VALU write needs before the swap reads it. Never pass an MFMA result.
+SJK_DEV void swap16(uint32_t & x, uint32_t & y) { asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(x), "+v"(y)); }
+SJK_DEV void swap32(uint32_t & x, uint32_t & y) { asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(x), "+v"(y)); }
+
 // ---- the host's NaN rule, for the paths that see non-finite values ----
 // A stored NaN half keeps only its sign (sign | 0x7E00), so the sign of every NaN the arithmetic makes is part
 // of the bytes. IEEE 754 leaves it unspecified; the reference's host build (x86-64 SSE) returns a quieted copy of

@@ -28,13 +28,6 @@ SJK_DEV u2 split2(float x0, float x1) {
               (uint32_t) __builtin_bit_cast(uint16_t, c) | ((uint32_t) __builtin_bit_cast(uint16_t, d) << 16)};
 }
 
-// Row exchange between two registers: v_permlane16_swap_b32 swaps the odd 16-lane rows of x with the even
-// rows of y, v_permlane32_swap_b32 the upper 32 lanes of x with the lower 32 of y (no LDS round trip, unlike
-// a lane shuffle). Written out as asm because this toolchain's builtin returns the first register for both
-// results; s_nop 1 gives the wait states a VALU write needs before the swap reads it. Never pass an MFMA result.
-SJK_DEV void swap16(uint32_t & x, uint32_t & y) { asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(x), "+v"(y)); }
-SJK_DEV void swap32(uint32_t & x, uint32_t & y) { asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(x), "+v"(y)); }
-
 // sum / max over the four 16-lane rows of a wavefront (the MFMA lane groups g), (r0 + r1) + (r2 + r3), the
 // same value in every lane
 SJK_DEV float rows_sum(float v) {

@@ -77,6 +77,10 @@ struct RowBatch {
 
 static_assert(sizeof(RowBatch) <= 4096, "the job table travels in the kernel arguments");
 
+template <int CTRL> SJK_DEV float dpp(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+}
+
 // Hadamard of one row held V values per lane (sj_kvarn.h:735-752): stages h < V inside the lane, stages h >= V
 // between lanes l and l ^ (h / V) (the lower partner keeps a + b, the upper a - b, a = the lower value), then one
 // multiply by 1/sqrt(D). XN: the host's NaN rule (a row holding an infinity or a NaN).
@@ -91,13 +95,43 @@ SJK_DEV void hadamard_row(float (&x)[V], int lane, float scale) {
                 x[m] = XN ? xadd(a, b) : a + b;
                 x[m + h] = XN ? xsub(a, b) : a - b;
             }
+    if (XN) {
 #pragma unroll
-    for (int lm = 1; lm < 64; lm *= 2) {
-        const bool upper = (lane & lm) != 0;
+        for (int lm = 1; lm < 64; lm *= 2) {
+            const bool upper = (lane & lm) != 0;
 #pragma unroll
-        for (int m = 0; m < V; ++m) {
-            const float o = __shfl_xor(x[m], lm, 64);
-            x[m] = upper ? (XN ? xsub(o, x[m]) : o - x[m]) : (XN ? xadd(x[m], o) : x[m] + o);
+            for (int m = 0; m < V; ++m) {
+                const float o = __shfl_xor(x[m], lm, 64);
+                x[m] = upper ? xsub(o, x[m]) : xadd(x[m], o);
+            }
+        }
+    } else {
+        // the partners' values by DPP inside a 16-lane row, then by row swaps: none of a lane shuffle's LDS round trips
+        // (six one after the other; appends of 8 rows at D = 256 4.5 -> 4.3 us, of 8,192 9.2 -> 8.7, fp16 rows 2.85 -> 2.63
+        // and 5.1 -> 4.95)
+        auto stage = [&](int lm, auto && partner) {
+            const bool upper = (lane & lm) != 0;
+#pragma unroll
+            for (int m = 0; m < V; ++m) {
+                const float o = partner(x[m]);
+                x[m] = upper ? o - x[m] : x[m] + o;
+            }
+        };
+        stage(1, [](float v) { return dpp<0xB1>(v); });                 // quad_perm 1 0 3 2
+        stage(2, [](float v) { return dpp<0x4E>(v); });                 // quad_perm 2 3 0 1
+        stage(4, [](float v) { return dpp<0x1B>(dpp<0x141>(v)); });     // 7 - l (row_half_mirror), then quad_perm 3 2 1 0
+        stage(8, [](float v) { return dpp<0x128>(v); });                // row_ror 8
+#pragma unroll
+        for (int lm = 16; lm < 64; lm *= 2) {
+            const bool upper = (lane & lm) != 0;
+#pragma unroll
+            for (int m = 0; m < V; ++m) {
+                uint32_t lo = f_bits(x[m]), hi = lo;                    // the lower and the upper partner's value
+                if (lm == 16) swap16(lo, hi);
+                else swap32(lo, hi);
+                const float p = __builtin_bit_cast(float, lo), q = __builtin_bit_cast(float, hi);
+                x[m] = upper ? p - q : p + q;
+            }
         }
     }
 #pragma unroll
