@@ -14,10 +14,14 @@
 // (a segment) into one part per wavefront. A wavefront is on its own from the query rows' staging to the segment's merge.
 // A tile cut over several workgroups is put together by prefill_combine; the first segment's O waits in the output.
 //
-// Numerics as the 16-row kernels: records enter as exact codes (fp16 subnormals c x 2^-24), Q' = Q x Kscale in fp16 hi + lo
-// parts, P' = P x Vscale x 2^k rounded to fp16 once, zero points and sums in fp32. Staged rows: a tq6_0 value enters as
-// the fp16 hi + lo parts of its centroid, the K block norm multiplies the fp32 sum of its block, the V block norm the
-// weight P, which is split hi + lo: three products each.
+// Numerics as the 16-row kernels. Records enter as exact codes (fp16 subnormals c x 2^-24); Q' = Q x Kscale is split into
+// fp16 hi + lo parts from the 32-bit query's exact product, zero points and sums are fp32, P' = P x Vscale x 2^k is rounded to
+// fp16 once (against the record's own maximum, where those take the running one). Staged rows: the query enters as fp16
+// hi + lo parts (times a power of two per row, so that a large row does not overflow and a small one does not lose its low
+// part), a tq6_0 value as the hi + lo parts of its centroid, the K block norm multiplies the fp32 sum of its block, the V
+// block norm the weight P, which is split hi + lo: three products each. Error against float64 at 7K-20K positions 0.88-1.12
+// of the 16-row kernels'. Q' from a query cut to fp16 parts first took 1% less time, but was off by 8e-3 on rows whose
+// channels are 2^20 apart and up to 1.1x further off than now with Kscale near 2^-9.
 //
 // What bounds it (D = 256): vector issue. A record is 128 + 64 products of 32 cycles, 6,100 cycles of a SIMD's matrix
 // core, and about 2,300 vector instructions, 10,000 cycles at their measured 2.5-5 each; 32 staged positions 96
@@ -35,7 +39,7 @@ constexpr int PF_ROWS = 32;                      // query rows of a tile: the co
 constexpr int PF_NW = 8, PF_NT = 64 * PF_NW;
 constexpr int PF_CH = 32;                        // staged positions per step
 constexpr int PF_MSTR = 68;                      // floats per query row of a merge slice (64 channels, 16-byte rows)
-constexpr int PF_WAVE = PF_ROWS * PF_MSTR * 4;   // LDS bytes per wavefront
+constexpr int PF_WAVE = PF_CH * 200;             // LDS bytes per wavefront: staged V rows and K norms
 
 // cost of 32 staged positions and of a sealed record: 3 : 4 was the fastest; 7 : 10 took 2% longer, 2 : 3 1.5% and 5 : 9 8% on
 // the 32K ubatch above
@@ -72,10 +76,16 @@ typedef uint32_t u4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 
 template <int D> struct PreLds {
     u2 pt[4096];                                 // tq6_0 pair table (fp16 hi, lo pairs)
-    alignas(16) uint16_t q[2][PF_ROWS][D + 8];   // Q hi / lo (row stride 16 bytes off the banks' period)
-    alignas(16) uint8_t wv[PF_NW][PF_WAVE];      // per wavefront: record scales, staged V rows, merge slices
+    union {
+        struct {                                 // (row strides 16 bytes off the banks' period)
+            alignas(16) float qf[PF_ROWS][D + 4];          // Q, for the records
+            alignas(16) uint16_t q[2][PF_ROWS][D + 8];     // Q hi / lo, for the staged rows
+            alignas(16) uint8_t wv[PF_NW][PF_WAVE];        // per wavefront: record scales, staged V rows
+        };
+        alignas(16) float mg[PF_NW][PF_ROWS * PF_MSTR];    // merge slices: the segment's rows are done with
+    };
     float wm[PF_NW][PF_ROWS], wl[PF_NW][PF_ROWS];
-    float rs[PF_ROWS];
+    float rs[PF_ROWS];                           // what takes a staged row's scores back to log2 units
     float cent[64];
 };
 
@@ -196,6 +206,15 @@ SJK_DEV void pin(float & v) { asm volatile("" : "+v"(v)); }
 SJK_DEV int fresh(int v) { asm volatile("" : "+v"(v)); return v; }
 SJK_DEV void pin(f16v & v) { asm volatile("" : "+v"(v)); }
 SJK_DEV void pin(uint32_t & v) { asm volatile("" : "+v"(v)); }
+// (a0 * s.lo, a1 * s.hi) as fp16 pairs {hi, lo}: hi = RN16(x), lo = RN16(x - hi) of the exact products x, by v_fma_mixlo /
+// mixhi (z = -0 as for mix_lo). Plain code, not the asm of the 16-row kernels: the compiler places the wait states
+// before the MFMAs that read the pairs, and moves other instructions into them
+SJK_DEV u2 mul_split(float a0, float a1, uint32_t s, float z) {
+    uint32_t h = __builtin_bit_cast(uint32_t, h2v{(_Float16) mix_lo(a0, s, z), (_Float16) mix_hi(a1, s, z)});
+    pin(h);                                      // one register: its halves are read in place
+    return u2{h, __builtin_bit_cast(uint32_t, h2v{(_Float16) fma_lo(a0, s, -h2f(h & 0xFFFFu)), (_Float16) fma_hi(a1, s, -h2f(h >> 16))})};
+}
+
 // HBM -> LDS without registers: lane l's word to dst + size x l
 SJK_DEV void dma4(gptr src, uint8_t * dst) {
     __builtin_amdgcn_global_load_lds((const void *) src, (__attribute__((address_space(3))) void *) dst, 4, 0, 0);
@@ -211,7 +230,7 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
     constexpr int NB = D / 128, NT = D / 32, NC = D / 16;        // tq6_0 blocks of a row, O tiles, K steps
     using RL4 = RecLay<4, 4, D>;
     constexpr int SC_BYTES = RL4::BYTES - RL4::KSC;              // a record's scale tables
-    static_assert(2 * SC_BYTES <= PF_WAVE && 32 * 196 + 32 * 2 * NB <= PF_WAVE, "a wavefront's LDS");
+    static_assert(2 * SC_BYTES <= PF_WAVE && PF_CH * 196 + PF_CH * 2 * NB <= PF_WAVE, "a wavefront's LDS");
     __shared__ PreLds<D> L;
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -244,9 +263,10 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
         const uint32_t left = (uint32_t) (xe - x < (uint64_t) (c.cost - from) ? xe - x : (uint64_t) (c.cost - from));
         const uint32_t to = from + left;
         const int r0 = PF_ROWS * tile, nr = a.rows - r0 < PF_ROWS ? a.rows - r0 : PF_ROWS;
-        // the query rows as fp16 hi + lo parts, each row scaled by a power of two to a largest value in [2, 4); rs gives the
-        // scores their scale back and is positive (a negative scale negates the row, a zero one clears it), so that the
-        // largest score is the largest product
+        // the query rows: as they are for the records (a negative scale negates the row, a zero one clears it, so that the
+        // largest score is the largest product), and for the staged rows as fp16 hi + lo parts of the row times the power
+        // of two that takes its largest value to [2^14, 2^15): channels down to 2^-28 of it keep 22 bits, as every channel
+        // of the records' 32-bit rows keeps its own
         __syncthreads();
         {
             const int tid = fresh((int) threadIdx.x);
@@ -264,7 +284,9 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
                 mx = fmaxf(mx, fabsf(xv[k]));
             }
             mx = row_max(mx);
-            const int e = mx > 0.0f && mx < 3e38f ? 2 - __builtin_amdgcn_frexp_expf(mx) : 0;
+            const int e = mx > 0.0f && mx < __builtin_inff() ? 15 - __builtin_amdgcn_frexp_expf(mx) : 0;
+#pragma unroll
+            for (int k = 0; k < PT; k += 4) *(float4 *) &L.qf[r][c0 + k] = *(const float4 *) &xv[k];
 #pragma unroll
             for (int k = 0; k < PT; k += 2) {
                 const u2 hl = split_pk(__builtin_amdgcn_ldexpf(xv[k], e), __builtin_amdgcn_ldexpf(xv[k + 1], e));
@@ -634,42 +656,26 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
                     for (int e = 0; e < 2; ++e)
 #pragma unroll
                         for (int i = 0; i < 16; ++i) S[u][e][i] = 0.0f;
-                f4 corr = {0.0f, 0.0f, 0.0f, 0.0f};
+                float corr = 0.0f;               // sum over this lane's channels of Q x Kzero
 #pragma unroll
                 for (int ck = 0; ck < NC; ++ck) {
-                    u4 qh, ql, ks, kz;
+                    u4 Bh, Bl;
                     {
-                        const u2 a0 = *(const u2 *) &L.q[0][m][16 * ck + 4 * h], a1 = *(const u2 *) &L.q[0][m][16 * ck + 8 + 4 * h];
-                        const u2 b0 = *(const u2 *) &L.q[1][m][16 * ck + 4 * h], b1 = *(const u2 *) &L.q[1][m][16 * ck + 8 + 4 * h];
-                        qh = u4{a0.x, a1.x, a0.y, a1.y};
-                        ql = u4{b0.x, b1.x, b0.y, b1.y};
+                        const f4 x0 = *(const f4 *) &L.qf[m][16 * ck + 4 * h], x1 = *(const f4 *) &L.qf[m][16 * ck + 8 + 4 * h];
                         const uint8_t * kp = sc0 + 2 * (2 * h * (D / 4) + 4 * ck);
                         const u2 s0 = *(const u2 *) kp, s1 = *(const u2 *) (kp + D / 2);
                         const u2 z0 = *(const u2 *) (kp + KZE), z1 = *(const u2 *) (kp + KZE + D / 2);
-                        ks = u4{s0.x, s0.y, s1.x, s1.y};
-                        kz = u4{z0.x, z0.y, z1.x, z1.y};
-                    }
-                    // Q' = Q x Kscale as hi + lo parts: hi = RN(Qh s), lo = RN(Ql s + (Qh s - hi)), the bracket exact
-                    u4 Bh, Bl;
+                        const float q[8] = {x0[0], x0[1], x1[0], x1[1], x0[2], x0[3], x1[2], x1[3]};
+                        const uint32_t ks[4] = {s0.x, s0.y, s1.x, s1.y}, kz[4] = {z0.x, z0.y, z1.x, z1.y};
+                        // Q' = Q x Kscale as hi + lo parts of the exact product
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const h2v q2 = __builtin_bit_cast(h2v, (uint32_t) qh[i]), l2 = __builtin_bit_cast(h2v, (uint32_t) ql[i]),
-                                  s2 = __builtin_bit_cast(h2v, (uint32_t) ks[i]);
-                        const h2v hi = q2 * s2;
-                        const h2v lo = __builtin_elementwise_fma(l2, s2, __builtin_elementwise_fma(q2, s2, -hi));
-                        Bh[i] = __builtin_bit_cast(uint32_t, hi);
-                        Bl[i] = __builtin_bit_cast(uint32_t, lo);
-                    }
-                    // sum over this lane's channels of Q x Kzero: 4x4x4 products whose A rows are all Kzero
-                    {
-                        const u2 zA = {kz.x, kz.y}, zB = {kz.z, kz.w};
-                        auto m4 = [&](const u2 & A, const u2 & B) {
-                            corr = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(h4, A), __builtin_bit_cast(h4, B), corr, 0, 0, 0);
-                        };
-                        m4(zA, u2{qh.x, qh.y});
-                        m4(zB, u2{qh.z, qh.w});
-                        m4(zA, u2{ql.x, ql.y});
-                        m4(zB, u2{ql.z, ql.w});
+                        for (int i = 0; i < 4; ++i) {
+                            const u2 hl = mul_split(q[2 * i], q[2 * i + 1], ks[i], nz);
+                            Bh[i] = hl.x;
+                            Bl[i] = hl.y;
+                            corr = fma_lo(q[2 * i], kz[i], corr);
+                            corr = fma_hi(q[2 * i + 1], kz[i], corr);
+                        }
                     }
                     u4 A[2][2];
 #pragma unroll
@@ -691,7 +697,7 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
                     SJK_FENCE();
                 }
                 __builtin_amdgcn_s_setprio(0);
-                const float ck = half_sum(corr[0] + 0.0f);
+                const float ck = half_sum(corr);
                 // scores; token of S[u][e][i]: 64 u + 16 (i / 4) + 8 e + 4 h + i % 4
                 float mx = -__builtin_inff();
                 const bool edge = p0 + 128u > qend_min;
@@ -712,7 +718,7 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
                             }
                             if (i4 & 1) SJK_FENCE();
                         }
-                const float rs = L.rs[m];
+                const float rs = a.sc2 == 0.0f ? 1.0f : fabsf(a.sc2);
                 if (edge) {
                     const uint32_t qend = q_end(m);
                     mx = -__builtin_inff();
@@ -836,7 +842,7 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
             const float inv = whole ? (ls == 0.0f ? 0.0f : 1.0f / ls) : 1.0f;
 #pragma unroll
             for (int p = 0; p < NT / 2; ++p) {
-                float * my = (float *) wv + m * PF_MSTR + 4 * h;
+                float * my = L.mg[w] + m * PF_MSTR + 4 * h;
 #pragma unroll
                 for (int e = 0; e < 2; ++e)
 #pragma unroll
@@ -846,7 +852,7 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
                 f4 y = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int k = 0; k < PF_NW; ++k) {
-                    const f4 z = *(const f4 *) ((const float *) L.wv[k] + r * PF_MSTR + 4 * c4);
+                    const f4 z = *(const f4 *) (L.mg[k] + r * PF_MSTR + 4 * c4);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) y[i] = __builtin_fmaf(fac[k], z[i], y[i]);
                 }

@@ -371,3 +371,68 @@ def test_prefill_kernel_edges(oracle, lib, dev, D, H, gq, n_q, staging, sink_typ
     finally:
         oracle.layer_free(C.byref(OL))
         lib.sj_kvarn_layer_free(C.byref(PL))
+
+
+def filled_context(lib, dev, OL, view, K, V, B, rotate=1):
+    """K, V rows [n][H][D] stored and [S, B) sealed in windows that fit the ring, the oracle's layer given the bytes"""
+    n_pos, H, D = K.shape
+    S, G, cfg = view.S, 128, OL.cfg
+    dK, dV = dev.put(K), dev.put(V)
+    done = S
+    for p in range(0, n_pos, 256):
+        n = min(256, n_pos - p)
+        at = lambda d: C.c_void_p(d.value + 4 * p * H * D)
+        sjk.check(lib.sjk_hip_layer_store(C.byref(view), p, n, at(dK), at(dV), rotate, None), "layer_store")
+        full = min(B, S + (p + n - S) // G * G) if p + n > S else S
+        if full > done:
+            sjk.check(lib.sjk_hip_commit(C.byref(view), 1, done, full, 16, None), "commit")
+            done = full
+    assert done == B
+    dev.sync()
+    sink_b = S * H * (4 * D if cfg.sink_type == 0 else 2 * OL.stage_bytes)
+    for name, nb in (("sink", sink_b), ("ring", OL.cap * H * 2 * OL.stage_bytes), ("body", (B - S) // G * H * OL.lay.bytes)):
+        if nb:
+            b = dev.get(C.c_void_p(getattr(view, name)), nb, np.uint8)
+            C.memmove(getattr(OL, name), b.ctypes.data, nb)
+
+
+def some_rows(n_q, n_head, n, seed):
+    rng = np.random.default_rng(seed)
+    return sorted({(0, 0), (1, n_head - 1), (n_q - 1, 0), (n_q - 1, n_head - 1)} |
+                  {(int(a), int(b)) for a, b in zip(rng.integers(0, n_q, n), rng.integers(0, n_head, n))})
+
+
+@pytest.mark.parametrize("D", [256, 128])
+def test_prefill_query_keeps_its_32_bits(oracle, lib, dev, D):
+    """A query row with one channel of 2^15 and the others of about 2^-5 (a ratio of 2^20), against keys that weigh them
+    alike: every channel's own relative precision counts, so a query cut to parts that share the row's largest exponent
+    loses the small channels (an error of 8e-3 in the values). Bound: the one 16-bit rounding in the path is that of P'
+    (2^-11 of a weight), and the code x Vscale it multiplies has about 3.2 times the size of the value it makes (codes 0
+    to 15, a zero point in the middle): errors that add up like the values themselves stay below 3.2 x 2^-11 of a row's
+    norm. The 16-row kernels' result for the same call (output over the queries) is held to the same."""
+    H, gq, n_q, S, ngr = 2, 4, 64, 128, 9
+    B = S + 128 * ngr
+    n_pos = B + 301
+    OL, PL = make_pair(oracle, lib, D, H, 4, 4, 0, 256, 512, n_ctx=4096, n_ubatch=512, staging=1)
+    view = lib.sjk_layer_view(C.byref(PL))
+    try:
+        rng = np.random.default_rng(500 + D)
+        K = 32.0 * rng.standard_normal((n_pos, H, D), dtype=np.float32)
+        K[:, :, 7] *= np.float32(2.0 ** -20)
+        V = rng.standard_normal((n_pos, H, D), dtype=np.float32)
+        filled_context(lib, dev, OL, view, K, V, B, rotate=0)
+        q = np.float32(2.0 ** -5) * rng.standard_normal((n_q, H * gq, D), dtype=np.float32)
+        q[:, :, 7] = np.where(rng.integers(0, 2, (n_q, H * gq)), 40000.0, -36000.0)
+        scale = 1.0 / float(np.sqrt(D))
+        got = attend(lib, dev, view, B, n_pos, n_pos - n_q, q, scale)
+        want = oracle_rows(oracle, OL, B, n_pos, q, n_pos - n_q, scale, some_rows(n_q, H * gq, 60, 8))
+        dq = dev.put(q)
+        sjk.check(lib.sjk_hip_attend(C.byref(view), B, n_pos, n_pos - n_q, n_q, H * gq, dq, scale, dq, None), "attend over q")
+        for name, x in (("32", got), ("16", dev.get(dq, q.nbytes, np.float32).reshape(q.shape))):
+            worst, l2 = check_rows(x, want)
+            say("[tiles] prefill D=%d, channels 2^20 apart, %s-row kernel: worst %.4f of the tolerance, rel L2 %.2e" % (
+                D, name, worst, l2))
+            assert l2 <= 3.2 * 2.0 ** -11
+    finally:
+        oracle.layer_free(C.byref(OL))
+        lib.sj_kvarn_layer_free(C.byref(PL))
