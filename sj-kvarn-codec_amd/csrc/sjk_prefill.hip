@@ -293,7 +293,12 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
                 *(uint32_t *) &L.q[0][r][c0 + k] = hl.x;
                 *(uint32_t *) &L.q[1][r][c0 + k] = hl.y;
             }
-            if ((tid & 15) == 0) L.rs[r] = a.sc2 == 0.0f ? 1.0f : __builtin_amdgcn_ldexpf(fabsf(a.sc2), -e);
+            if ((tid & 15) == 0) {
+                // never 0, which would make a NaN of a masked score (0 x -inf): a row so small that its factor is below the
+                // smallest normal number has scores below 2^-80 with that number too, and weights of exactly 1
+                const float f = a.sc2 == 0.0f ? 1.0f : __builtin_amdgcn_ldexpf(fabsf(a.sc2), -e);
+                L.rs[r] = f < 0x1p-126f ? 0x1p-126f : f;
+            }
         }
         __syncthreads();
         // the visible end of query row m (0: none for a dead row), computed where it is needed

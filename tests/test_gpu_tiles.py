@@ -436,3 +436,29 @@ def test_prefill_query_keeps_its_32_bits(oracle, lib, dev, D):
     finally:
         oracle.layer_free(C.byref(OL))
         lib.sj_kvarn_layer_free(C.byref(PL))
+
+
+@pytest.mark.parametrize("D,staging", [(256, 0), (128, 1)])
+def test_prefill_tiny_queries_and_scales(oracle, lib, dev, D, staging):
+    """Scores that round to zero: subnormal query rows, and a scale whose product with the row is below every float.
+    The rows are plain means over what they see, positions that a row does not see stay out of it."""
+    H, gq, n_q, S = 2, 4, 64, 128
+    B = S + 3 * 128
+    n_pos = B + 301
+    OL, PL = make_pair(oracle, lib, D, H, 4, 4, 0, 256, 512, n_ctx=4096, n_ubatch=512, staging=staging)
+    view = lib.sjk_layer_view(C.byref(PL))
+    try:
+        K, V = inputs.kv_rows(n_pos, H, D, seed=91)
+        filled_context(lib, dev, OL, view, K, V, B)
+        for name, amp, scale in (("subnormal rows", 1e-44, 0.0625), ("1e-30 rows", 1e-30, -0.0625),
+                                 ("subnormal scale", 0.25, 1e-45), ("rows and scale", 1e-25, 1e-25)):
+            q = np.float32(amp) * np.random.default_rng(4).uniform(0.5, 1.0, (n_q, H * gq, D)).astype(np.float32)
+            q[3] = 0.0
+            for qpos0 in (n_pos - n_q, B - 40, 20):          # rows in the tail, across the body's end, in the sink
+                got = attend(lib, dev, view, B, n_pos, qpos0, q, scale)
+                assert np.isfinite(got).all(), (name, qpos0)
+                worst, _ = check_rows(got, oracle_rows(oracle, OL, B, n_pos, q, qpos0, scale, some_rows(n_q, H * gq, 20, 5)))
+                say("[tiles] prefill D=%d %s at %d: worst %.4f of the tolerance" % (D, name, qpos0, worst))
+    finally:
+        oracle.layer_free(C.byref(OL))
+        lib.sj_kvarn_layer_free(C.byref(PL))
