@@ -86,6 +86,7 @@ template <int D> struct PreLds {
     };
     float wm[PF_NW][PF_ROWS], wl[PF_NW][PF_ROWS];
     float rs[PF_ROWS];                           // what takes a staged row's scores back to log2 units
+    uint32_t see[PF_ROWS];                       // the visible end of a query row (0: none for a dead row)
     float cent[64];
 };
 
@@ -100,9 +101,9 @@ SJK_DEV u2 split_pk(float a, float b) {          // (a, b) as fp16 pairs {hi, lo
     const h2v h = __builtin_bit_cast(h2v, hi);
     return u2{hi, pk16(a - (float) h[0], b - (float) h[1])};
 }
-// fp32 times the low / high fp16 half of h: with z = -0 in a register one v_fma_mix (else a conversion and a product)
-SJK_DEV float mix_lo(float a, uint32_t h, float z) { return __builtin_fmaf(a, h2f(h & 0xFFFFu), z); }
-SJK_DEV float mix_hi(float a, uint32_t h, float z) { return __builtin_fmaf(a, h2f(h >> 16), z); }
+// fp32 times the low / high fp16 half of h: plus 0, so that it is one v_fma_mix (else a conversion and a product)
+SJK_DEV float mix_lo(float a, uint32_t h) { return __builtin_fmaf(a, h2f(h & 0xFFFFu), 0.0f); }
+SJK_DEV float mix_hi(float a, uint32_t h) { return __builtin_fmaf(a, h2f(h >> 16), 0.0f); }
 
 // over the wavefront's halves, the same value in both (never of an MFMA's result itself, see swap32)
 SJK_DEV float half_sum(float v) {
@@ -207,14 +208,16 @@ SJK_DEV int fresh(int v) { asm volatile("" : "+v"(v)); return v; }
 SJK_DEV void pin(f16v & v) { asm volatile("" : "+v"(v)); }
 SJK_DEV void pin(uint32_t & v) { asm volatile("" : "+v"(v)); }
 // (a0 * s.lo, a1 * s.hi) as fp16 pairs {hi, lo}: hi = RN16(x), lo = RN16(x - hi) of the exact products x, by v_fma_mixlo /
-// mixhi (z = -0 as for mix_lo). Plain code, not the asm of the 16-row kernels: the compiler places the wait states
+// mixhi. Plain code, not the asm of the 16-row kernels: the compiler places the wait states
 // before the MFMAs that read the pairs, and moves other instructions into them
-SJK_DEV u2 mul_split(float a0, float a1, uint32_t s, float z) {
-    uint32_t h = __builtin_bit_cast(uint32_t, h2v{(_Float16) mix_lo(a0, s, z), (_Float16) mix_hi(a1, s, z)});
+SJK_DEV u2 mul_split(float a0, float a1, uint32_t s) {
+    uint32_t h = __builtin_bit_cast(uint32_t, h2v{(_Float16) mix_lo(a0, s), (_Float16) mix_hi(a1, s)});
     pin(h);                                      // one register: its halves are read in place
     return u2{h, __builtin_bit_cast(uint32_t, h2v{(_Float16) fma_lo(a0, s, -h2f(h & 0xFFFFu)), (_Float16) fma_hi(a1, s, -h2f(h >> 16))})};
 }
 
+// bit 15 / 31: the low / high half is an infinity or a NaN
+SJK_DEV uint32_t nonfinite_halves(uint32_t w) { return ((w & 0x7FFF7FFFu) + 0x04000400u) & 0x80008000u; }
 // HBM -> LDS without registers: lane l's word to dst + size x l
 SJK_DEV void dma4(gptr src, uint8_t * dst) {
     __builtin_amdgcn_global_load_lds((const void *) src, (__attribute__((address_space(3))) void *) dst, 4, 0, 0);
@@ -268,6 +271,10 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
         // of two that takes its largest value to [2^14, 2^15): channels down to 2^-28 of it keep 22 bits, as every channel
         // of the records' 32-bit rows keeps its own
         __syncthreads();
+        if (tid < PF_ROWS) {
+            const uint32_t e = c.qpos0 + (uint32_t) ((r0 + tid) / a.gq) + 1u;
+            L.see[tid] = tid < nr ? (e < c.N ? e : c.N) : 0u;
+        }
         {
             const int tid = fresh((int) threadIdx.x);
             constexpr int PT = D / 16;           // values per thread, 16 threads a row
@@ -301,11 +308,6 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
             }
         }
         __syncthreads();
-        // the visible end of query row m (0: none for a dead row), computed where it is needed
-        auto q_end = [&](int m) {
-            const uint32_t e = c.qpos0 + (uint32_t) ((r0 + m) / a.gq) + 1u;
-            return m < nr ? (e < c.N ? e : c.N) : 0u;
-        };
         uint32_t qend_min = c.qpos0 + (uint32_t) (r0 / a.gq) + 1u;   // visible to every live row
         if (qend_min > c.N) qend_min = c.N;
 
@@ -479,12 +481,19 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
                         }
                     }
                     const float rs = L.rs[m];
-                    if (p1 - p0 < PF_CH || p1 > qend_min) {
-                        const uint32_t qend = q_end(m);
+                    // positions that the row does not see: no score, and nothing of their values, whose infinities and NaNs
+                    // would make a NaN with a weight of zero (dead: a bit per score)
+                    const bool edge = p1 - p0 < PF_CH || p1 > qend_min;
+                    uint32_t dead = 0;
+                    if (edge) {
+                        const uint32_t qend = L.see[m];
 #pragma unroll
                         for (int i = 0; i < 16; ++i) {
                             const uint32_t p = p0 + (uint32_t) (8 * (i >> 2) + 4 * h + (i & 3));
-                            if (p >= p1 || p >= qend) sc[i] = -__builtin_inff();
+                            if (p >= p1 || p >= qend) {
+                                sc[i] = -__builtin_inff();
+                                dead |= 1u << i;
+                            }
                         }
                     }
                     float mx = sc[0];
@@ -530,6 +539,15 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
                                 Ph[u] = hl.x;
                                 Pl[u] = hl.y;
                             }
+                            if (!F16 && edge) {
+#pragma unroll
+                                for (int u = 0; u < 4; ++u) {
+                                    const uint32_t d = dead >> (8 * s + 2 * u);
+                                    const uint32_t live = ((d & 1u) ? 0u : 0xFFFFu) | ((d & 2u) ? 0u : 0xFFFF0000u);
+                                    Ph[u] &= live;
+                                    Pl[u] &= live;
+                                }
+                            }
                             // per token the pair-table indices of channels 4 m, 4 m + 1 and 4 m + 2, 4 m + 3 (or the halves)
                             u2 ix[8];
 #pragma unroll
@@ -542,6 +560,44 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
                                     const uint32_t qs = *(const uint16_t *) (r + 2 + 2 * m), qh = r[66 + m];
                                     const uint32_t z = (qh | (qh << 4)) & 0x0F0Fu;
                                     ix[t].x = __builtin_amdgcn_perm(z, qs, 0x05010400u);
+                                }
+                            }
+                            // fp16 values are shared by the rows of a product: in a step that not every row sees whole, those
+                            // that are not finite leave it, and are added to the rows that see them (their weights go
+                            // through LDS, -1 for the others)
+                            if (F16 && edge) {
+                                h2v nf = {(_Float16) 0.0f, (_Float16) 0.0f};
+#pragma unroll
+                                for (int t = 0; t < 8; ++t)
+#pragma unroll
+                                    for (int k2 = 0; k2 < 2; ++k2)       // 0 x value: a NaN if it is not finite
+                                        nf = __builtin_elementwise_fma(__builtin_bit_cast(h2v, (uint32_t) ix[t][k2]), h2v{(_Float16) 0.0f, (_Float16) 0.0f}, nf);
+                                if (__builtin_expect(__any(nonfinite_halves(__builtin_bit_cast(uint32_t, nf)) != 0u), 0)) {
+                                    float * pw = (float *) wv + m;
+#pragma unroll
+                                    for (int t = 0; t < 8; ++t) {
+                                        ix[t].x &= ~((nonfinite_halves(ix[t].x) >> 15) * 0xFFFFu);
+                                        ix[t].y &= ~((nonfinite_halves(ix[t].y) >> 15) * 0xFFFFu);
+                                        pw[32 * (tok(t) - 16 * s)] = (dead >> (8 * s + t) & 1u) ? -1.0f : sc[8 * s + t];
+                                    }
+                                    wave_sync();
+#pragma unroll 1
+                                    for (uint32_t t = 0; t < 16u && p0 + 16u * s + t < p1; ++t) {
+                                        const float pt = pw[32 * t];
+                                        const gptr vr = row(p0 + 16u * s + t) + 2 * D + 2 * (128 * b + 16 * h);
+#pragma unroll
+                                        for (int i = 0; i < 16; ++i) {
+                                            const u2 x = gload<u2>(vr + 8 * (8 * (i >> 2) + (i & 3)));
+#pragma unroll
+                                            for (int jj = 0; jj < 4; ++jj) {
+                                                const uint32_t v = (x[jj >> 1] >> (16 * (jj & 1))) & 0xFFFFu;
+                                                if (nonfinite_halves(v) && !(pt < 0.0f)) O[4 * b + jj][i] += pt * h2f(v);
+                                            }
+                                        }
+                                    }
+#pragma unroll
+                                    for (int jj = 0; jj < 4; ++jj) pin(O[4 * b + jj]);
+                                    wave_sync();
                                 }
                             }
                             SJK_FENCE();
@@ -642,8 +698,7 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
             for (int ck = 0; ck < KD; ++ck) kload(rec, ck, lblk() * (uint32_t) (NC * 128) + lofs());
             for (int g = g0; g < g1; ++g) {
                 uint32_t M0 = 0x000F000Fu, M1 = 0x00F000F0u;     // in registers: an AND with a constant takes twice as long
-                float nz = -0.0f;
-                pin(M0); pin(M1); pin(nz);
+                pin(M0); pin(M1);
                 const int lane = fresh(tid) & 63, m = lane & 31, h = lane >> 5;
                 const uint32_t p0 = V.S + 128u * (uint32_t) g;
                 const uint8_t * sc0 = wv + ((g - g0) & 1) * SC_BYTES;
@@ -675,30 +730,25 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
                         // Q' = Q x Kscale as hi + lo parts of the exact product
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
-                            const u2 hl = mul_split(q[2 * i], q[2 * i + 1], ks[i], nz);
+                            const u2 hl = mul_split(q[2 * i], q[2 * i + 1], ks[i]);
                             Bh[i] = hl.x;
                             Bl[i] = hl.y;
                             corr = fma_lo(q[2 * i], kz[i], corr);
                             corr = fma_hi(q[2 * i + 1], kz[i], corr);
                         }
                     }
-                    u4 A[2][2];
 #pragma unroll
                     for (int u = 0; u < 2; ++u) {
                         const u2 k2 = kw[ck % KD][u];
                         const uint32_t x0 = k2.x, x1 = k2.x >> 8, y0 = k2.y, y1 = k2.y >> 8;
-                        A[u][0] = u4{x0 & M0, x1 & M0, y0 & M0, y1 & M0};
-                        A[u][1] = u4{x0 & M1, x1 & M1, y0 & M1, y1 & M1};
+                        const u4 A[2] = {u4{x0 & M0, x1 & M0, y0 & M0, y1 & M0}, u4{x0 & M1, x1 & M1, y0 & M1, y1 & M1}};
+#pragma unroll
+                        for (int e = 0; e < 2; ++e) S[u][e] = mfma3216(A[e], Bh, S[u][e]);
+                        if (u == 1 && ck + KD < NC) kload(rec, ck + KD, koff);
+#pragma unroll
+                        for (int e = 0; e < 2; ++e) S[u][e] = mfma3216(A[e], Bl, S[u][e]);
+                        if (u == 0) SJK_FENCE();
                     }
-#pragma unroll
-                    for (int u = 0; u < 2; ++u)
-#pragma unroll
-                        for (int e = 0; e < 2; ++e) S[u][e] = mfma3216(A[u][e], Bh, S[u][e]);
-                    if (ck + KD < NC) kload(rec, ck + KD, koff);
-#pragma unroll
-                    for (int u = 0; u < 2; ++u)
-#pragma unroll
-                        for (int e = 0; e < 2; ++e) S[u][e] = mfma3216(A[u][e], Bl, S[u][e]);
                     SJK_FENCE();
                 }
                 __builtin_amdgcn_s_setprio(0);
@@ -717,7 +767,7 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
 #pragma unroll
                             for (int i = 0; i < 4; ++i) {
                                 const float y = __builtin_fmaf(S[u][e][4 * i4 + i], e ? 0x1p20f : 0x1p24f, ck);
-                                const float s = (i & 1) ? mix_hi(y, kt[i >> 1], nz) : mix_lo(y, kt[i >> 1], nz);
+                                const float s = (i & 1) ? mix_hi(y, kt[i >> 1]) : mix_lo(y, kt[i >> 1]);
                                 S[u][e][4 * i4 + i] = s;
                                 mx = fmaxf(mx, s);
                             }
@@ -725,7 +775,8 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
                         }
                 const float rs = a.sc2 == 0.0f ? 1.0f : fabsf(a.sc2);
                 if (edge) {
-                    const uint32_t qend = q_end(m);
+                    const uint32_t qend = L.see[m];
+                    const int n_see = (int) (qend - p0);         // of the record's tokens
                     mx = -__builtin_inff();
 #pragma unroll
                     for (int u = 0; u < 2; ++u)
@@ -733,7 +784,7 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
                         for (int e = 0; e < 2; ++e)
 #pragma unroll
                             for (int i = 0; i < 16; ++i) {
-                                if (p0 + (uint32_t) (64 * u + 16 * (i >> 2) + 8 * e + 4 * h + (i & 3)) >= qend) S[u][e][i] = -__builtin_inff();
+                                if (64 * u + 16 * (i >> 2) + 8 * e + 4 * h + (i & 3) >= n_see) S[u][e][i] = -__builtin_inff();
                                 mx = fmaxf(mx, S[u][e][i]);
                             }
                 }
@@ -743,7 +794,7 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
                 const float m_rec = mx * rs, m_new = fmaxf(m_run, m_rec);
                 const bool any = m_rec != -__builtin_inff();
                 const float alpha = any ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.0f;
-                const float f = any ? __builtin_amdgcn_exp2f(m_rec - m_new) : 0.0f;
+                const float f = any ? __builtin_amdgcn_exp2f(m_rec - m_new) : -0.0f;
                 const float m_sub = any ? m_rec : 0.0f;
                 float pinv, ps = 0.0f, cv = 0.0f;
                 const float psc = pv_scale(sc0 + VSC, lane, pinv);
@@ -761,7 +812,13 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
 #pragma unroll
                         for (int i4 = 0; i4 < 4; ++i4) {
                             const int t0 = 64 * u + 16 * i4 + 8 * e + 4 * h;
-                            const u2 vs = *(const u2 *) (sc0 + VSC + 2 * t0), vz = *(const u2 *) (sc0 + VZE + 2 * t0);
+                            u2 vs = *(const u2 *) (sc0 + VSC + 2 * t0), vz = *(const u2 *) (sc0 + VZE + 2 * t0);
+                            if (edge) {          // no scale of a token that the row does not see: it may not be finite
+                                const int k = (int) (L.see[m] - p0) - t0;
+                                const u2 live = {(k > 0 ? 0xFFFFu : 0u) | (k > 1 ? 0xFFFF0000u : 0u), (k > 2 ? 0xFFFFu : 0u) | (k > 3 ? 0xFFFF0000u : 0u)};
+                                vs &= live;
+                                vz &= live;
+                            }
                             float y[4];
 #pragma unroll
                             for (int i = 0; i < 4; ++i) {
@@ -769,7 +826,7 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
                                 ps += pr;
                                 const float px = pr * psc;
                                 cv = (i & 1) ? fma_hi(px, vz[i >> 1], cv) : fma_lo(px, vz[i >> 1], cv);
-                                y[i] = (i & 1) ? mix_hi(px, vs[i >> 1], nz) : mix_lo(px, vs[i >> 1], nz);
+                                y[i] = (i & 1) ? mix_hi(px, vs[i >> 1]) : mix_lo(px, vs[i >> 1]);
                             }
                             uint32_t pa = pk16(y[0], y[1]), pb = pk16(y[2], y[3]);
                             pin(ps); pin(cv); pin(pa); pin(pb);
@@ -805,14 +862,17 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(2))) void
                             t = mfma3216(u4{v2.x & M, (v2.x >> 8) & M, v2.y & M, (v2.y >> 8) & M}, Pa[s], t);
                             SJK_FENCE();
                         }
-                        // channel of C row 4 h + i + 8 i4: 64 p + 16 i4 + 8 e + 4 h + i, its Vch at (4 h + i) D/8 + 8 p + 2 i4 + e
+                        // channel of C row 4 h + i + 8 i4: 64 p + 16 i4 + 8 e + 4 h + i, its Vch at (4 h + i) D/8 + 8 p + 2 i4 + e;
+                        // rows that see nothing of the record take nothing, whatever its channel scales are
+                        if ((int) f_bits(f) >= 0) {              // not the -0 of such a row
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const u4 vc = *(const u4 *) (sc0 + VCH + 2 * ((4 * h + i) * (D / 8) + 8 * p));
+                            for (int i = 0; i < 4; ++i) {
+                                const u4 vc = *(const u4 *) (sc0 + VCH + 2 * ((4 * h + i) * (D / 8) + 8 * p));
 #pragma unroll
-                            for (int i4 = 0; i4 < 4; ++i4) {
-                                const float vcs = e ? mix_hi(pe, vc[i4], nz) : mix_lo(pe, vc[i4], nz);
-                                O[2 * p + e][4 * i4 + i] = __builtin_fmaf(t[4 * i4 + i] + cs, vcs, O[2 * p + e][4 * i4 + i]);
+                                for (int i4 = 0; i4 < 4; ++i4) {
+                                    const float vcs = e ? mix_hi(pe, vc[i4]) : mix_lo(pe, vc[i4]);
+                                    O[2 * p + e][4 * i4 + i] = __builtin_fmaf(t[4 * i4 + i] + cs, vcs, O[2 * p + e][4 * i4 + i]);
+                                }
                             }
                         }
                         pin(O[2 * p + e]);

@@ -410,7 +410,7 @@ def test_prefill_query_keeps_its_32_bits(oracle, lib, dev, D):
     (2^-11 of a weight), and the code x Vscale it multiplies has about 3.2 times the size of the value it makes (codes 0
     to 15, a zero point in the middle): errors that add up like the values themselves stay below 3.2 x 2^-11 of a row's
     norm. The 16-row kernels' result for the same call (output over the queries) is held to the same."""
-    H, gq, n_q, S, ngr = 2, 4, 64, 128, 9
+    H, gq, n_q, S, ngr = 2, 4, 72, 128, 9
     B = S + 128 * ngr
     n_pos = B + 301
     OL, PL = make_pair(oracle, lib, D, H, 4, 4, 0, 256, 512, n_ctx=4096, n_ubatch=512, staging=1)
@@ -442,7 +442,7 @@ def test_prefill_query_keeps_its_32_bits(oracle, lib, dev, D):
 def test_prefill_tiny_queries_and_scales(oracle, lib, dev, D, staging):
     """Scores that round to zero: subnormal query rows, and a scale whose product with the row is below every float.
     The rows are plain means over what they see, positions that a row does not see stay out of it."""
-    H, gq, n_q, S = 2, 4, 64, 128
+    H, gq, n_q, S = 2, 4, 72, 128
     B = S + 3 * 128
     n_pos = B + 301
     OL, PL = make_pair(oracle, lib, D, H, 4, 4, 0, 256, 512, n_ctx=4096, n_ubatch=512, staging=staging)
@@ -459,6 +459,61 @@ def test_prefill_tiny_queries_and_scales(oracle, lib, dev, D, staging):
                 assert np.isfinite(got).all(), (name, qpos0)
                 worst, _ = check_rows(got, oracle_rows(oracle, OL, B, n_pos, q, qpos0, scale, some_rows(n_q, H * gq, 20, 5)))
                 say("[tiles] prefill D=%d %s at %d: worst %.4f of the tolerance" % (D, name, qpos0, worst))
+    finally:
+        oracle.layer_free(C.byref(OL))
+        lib.sj_kvarn_layer_free(C.byref(PL))
+
+
+@pytest.mark.parametrize("D,staging,sink_type", [(256, 0, 0), (128, 0, 1), (256, 1, 1), (128, 1, 0)])
+def test_prefill_unseen_values_stay_out(oracle, lib, dev, D, staging, sink_type):
+    """An infinity or a NaN among the values of one position: the rows before it, whose weight for it is zero, keep
+    their bits (a product of zero with it would be a NaN); the rows that see it are not finite. The position is in the
+    sink, in the tail, or in a record (its value scale or zero point, or a channel's scale, which all tokens share)."""
+    H, gq, n_q, S = 2, 4, 72, 128
+    B = S + 4 * 128
+    n_pos = B + 301
+    OL, PL = make_pair(oracle, lib, D, H, 4, 4, 0, 256, 512, n_ctx=4096, n_ubatch=512, staging=staging, sink_type=sink_type)
+    view = lib.sjk_layer_view(C.byref(PL))
+    lay = OL.lay
+    sb = OL.stage_bytes
+    try:
+        K, V = inputs.kv_rows(n_pos, H, D, seed=92)
+        filled_context(lib, dev, OL, view, K, V, B)
+        q = np.random.default_rng(6).standard_normal((n_q, H * gq, D)).astype(np.float32)
+        scale = 1.0 / float(np.sqrt(D))
+
+        def staged(base, entry):                     # the V row's first half of head 1: a block norm or a value
+            return base + entry * H * 2 * sb + 2 * sb + sb
+
+        def sink_at(p):
+            return p * H * 4 * D + 4 * D + 2 * D if sink_type == 0 else staged(0, p)
+
+        rec = ((2 * H + 1) * lay.bytes, S + 2 * 128)  # record 2 of head 1, its first position
+        cases = []                                   # (name, pointer, offset, qpos0, first position that may differ)
+        for bad in (29, 8):
+            cases.append(("sink %d" % bad, view.sink, sink_at(bad), 0, bad))
+        for qpos0 in (n_pos - n_q, n_pos - 2 * n_q):  # the end of a tile's steps, and not
+            p = qpos0 + 29
+            cases.append(("tail %d" % p, view.ring, staged(0, (p - S) % OL.cap), qpos0, p))
+        for what, off, p in (("scale", lay.v_scale + 2 * 7, rec[1] + 7), ("zero", lay.v_zero + 2 * 7, rec[1] + 7),
+                             ("channel", lay.v_ch + 2 * 5, rec[1])):
+            cases.append(("record " + what, view.body, rec[0] + off, rec[1] - 30, p))
+        for name, ptr, off, qpos0, first in cases:
+            good = attend(lib, dev, view, B, n_pos, qpos0, q, scale)
+            assert np.isfinite(good).all(), name
+            ptr = C.c_void_p(ptr)
+            old = dev.get(ptr, 2, np.uint16, off)
+            for half in (0x7C00, 0xFE00):
+                dev.upload(ptr, np.array([half], np.uint16), off)
+                got = attend(lib, dev, view, B, n_pos, qpos0, q, scale)
+                n = first - qpos0
+                a, b = got.view(np.uint32), good.view(np.uint32)
+                bad = [(iq, hq) for iq in range(n) for hq in range(H * gq) if not np.array_equal(a[iq, hq], b[iq, hq])]
+                assert not bad, (name, hex(half), len(bad), bad[:4])
+                assert np.array_equal(a[:, :gq], b[:, :gq]), name          # the other head
+                assert not np.isfinite(got[n:, gq:]).all(axis=-1).any(), (name, hex(half))
+            dev.upload(ptr, old, off)
+            say("[tiles] prefill D=%d staging %d, %s: %d positions keep their rows" % (D, staging, name, first - qpos0))
     finally:
         oracle.layer_free(C.byref(OL))
         lib.sj_kvarn_layer_free(C.byref(PL))
