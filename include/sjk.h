@@ -344,7 +344,8 @@ int sjk_hip_commit_dyn(const sjk_hip_view * views, int n_layers, const int32_t *
  * hq to KV head hq / (n_head / n_head_kv). Any n_q and n_head (a prefill ubatch as well as a decode step):
  * the n_q x n_head / n_head_kv query rows of a KV head are cut into tiles of 16 rows, and a launch takes up to
  * 8 jobs side by side (sharing its workgroups in proportion to their work; each job reads the context); a 4/4
- * call of 256 rows and more whose output does not lie over its queries runs in one launch of 32-row tiles. The
+ * call of more than 256 rows (or of 256 and 8 KV heads) whose output does not lie over its queries runs in one launch
+ * of 32-row tiles. The
  * partial results go to v->work (SJKVARN_ERR_ARG without one). Every layout a layer can have runs
  * on a matrix-core kernel; a hand-built view outside them (another group size, head dimension or record
  * layout) is refused with SJK_ERR_UNSUPPORTED and a message (sjk_last_error), as are the batched, no-alloc and

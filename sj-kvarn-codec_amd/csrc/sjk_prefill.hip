@@ -45,12 +45,14 @@ constexpr int PF_WAVE = PF_CH * 200;             // LDS bytes per wavefront: sta
 // the 32K ubatch above
 constexpr int PF_COST_CH = 3, PF_COST_REC = 4;
 
-// Calls with fewer query rows per KV head take the 16-row kernels. From 256 rows (which there take two launches) this
-// kernel is the faster one at every length measured: 4/4 at D = 256, 4 heads, 37.7 against 38.2 us at 600 positions, 110
-// against 169 at 33K; at D = 128, 2 heads, 26.8 against 28.2 and 48.5 against 62.2. At 128 rows it takes up to twice
-// as long on short contexts (36 against 20 us at 600 positions). The line is on the rows alone: a captured call does not
-// know its context.
-constexpr int PF_MIN_ROWS = 256;
+// Calls with fewer query rows per KV head take the 16-row kernels. Past 256 rows, where those take a third launch, this
+// kernel is the faster one at every length and head count measured (100-33K positions, 1-16 KV heads, D = 128 and 256):
+// 260 rows of 1 head, D = 256, 39.5 against 49.0 us at 1,500 positions, 59 against 77 at 33K; of 2 heads, D = 128, 27.2
+// against 36.8 at 700. At 256 rows, two launches there, it needs 8 KV heads to win or to draw: D = 128, 27.9 against 27.5 us
+// at 300 positions, 34.4 against 44.6 at 1,500, 112 against 273 at 33K (16 heads: 1.2-2.8x); with 4 heads and D = 256
+// it takes 38.1 against 35.3 us at 600 positions, with 1 head 38.5 against 32.0 at 1,500. At 128 rows it takes up to twice as
+// long on short contexts. The line is on rows and heads alone: a captured call does not know its context.
+constexpr int PF_MIN_ROWS = 256, PF_MIN_ROWS_HEADS = 8;
 
 struct PreArgs {
     sjk_hip_view v;
@@ -1009,7 +1011,8 @@ namespace sjk {
 // workgroup still reads queries (a call with out over q takes the 16-row kernels, which write after all reads).
 bool sjk_prefill_takes(const sjk_hip_view & v, int body, int n_q, int n_head, const float * d_q, const float * d_out) {
     const size_t row = (size_t) n_q * (size_t) n_head * (size_t) v.lay.D, W = (size_t) n_cus(), sf = ws_slot_floats(v.lay.D);
-    if (n_q * (n_head / v.n_head_kv) < PF_MIN_ROWS) return false;
+    const int rows = n_q * (n_head / v.n_head_kv);
+    if (rows < PF_MIN_ROWS || (rows == PF_MIN_ROWS && v.n_head_kv < PF_MIN_ROWS_HEADS)) return false;
     if (body != 44 || v.work_bytes < WS_PLAN_BYTES + ws_stage_bytes(v.lay.D, v.n_head_kv)) return false;
     if (d_q < d_out + row && d_out < d_q + row) return false;
     return W * PF_ROWS * (size_t) v.lay.D + W * PF_ROWS * 4 <= ws_part_slots(v) * sf;

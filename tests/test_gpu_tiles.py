@@ -308,19 +308,23 @@ def test_wide_rows_vs_oracle(oracle, lib, dev, D, H, bk, bv, body, n_q, n_head, 
 
 PREFILL = [
     # D, H, gq, n_q, staging, sink_type, sealed groups, tail, first query position before the end, scale
-    (256, 4, 4, 64, 0, 0, 9, 301, 64, 0.0625),     # 256 rows, the fewest; a tail that is no multiple of 32
+    (256, 4, 4, 64, 0, 0, 9, 301, 64, 0.0625),     # 256 rows of 4 heads (16-row kernels); a tail that is no multiple of 32
     (128, 4, 4, 67, 0, 0, 9, 256, 67, 0.08),       # a last tile of 12 rows
     (256, 1, 16, 17, 0, 0, 0, 0, 128, 0.0625),     # causal in a sink that is all there is
     (256, 2, 8, 33, 0, 1, 3, 470, 300, 0.0625),    # sink in the staging type, rows across the body's end
     (128, 2, 4, 100, 1, 0, 4, 290, 600, -0.05),    # fp16 staging, a negative scale, later records masked
     (256, 4, 4, 64, 1, 1, 2, 257, 64, 0.0),        # fp16 sink in the staging type, scale 0 (plain means)
-    (128, 16, 4, 65, 0, 0, 1, 260, 65, 0.08),      # more tiles than there are compute units
+    (128, 16, 4, 65, 0, 0, 1, 260, 65, 0.08),      # 16 heads: 144 tiles
+    (256, 8, 4, 64, 0, 0, 9, 301, 64, 0.0625),     # 256 rows, the fewest that the 32-row kernel takes (from 8 heads on)
+    (256, 4, 4, 66, 1, 1, 2, 257, 66, 0.0),        # fp16 sink in the staging type, scale 0, a last tile of 8 rows
+    (128, 16, 4, 160, 0, 0, 3, 300, 160, 0.08),    # 320 tiles: some whole in their workgroup, which normalises them
+    (128, 4, 8, 300, 0, 1, 3, 450, 400, 0.08),     # 75 tiles a head: past the first 64 of the search for a share's tile
 ]
 
 
 @pytest.mark.parametrize("D,H,gq,n_q,staging,sink_type,ngr,tail,back,scale", PREFILL)
 def test_prefill_kernel_edges(oracle, lib, dev, D, H, gq, n_q, staging, sink_type, ngr, tail, back, scale):
-    """Calls of 256 query rows per KV head and more: ragged tiles, every region and staging type, causal rows in each
+    """Calls of 256 query rows per KV head and more, most of them on the 32-row kernel: ragged tiles, every region and staging type, causal rows in each
     region, each against the oracle; the descriptor call gives the same bits, and a call whose output lies over its
     queries (which takes the 16-row kernels) agrees with the oracle too."""
     S, G = 128, 128
@@ -400,6 +404,31 @@ def some_rows(n_q, n_head, n, seed):
     rng = np.random.default_rng(seed)
     return sorted({(0, 0), (1, n_head - 1), (n_q - 1, 0), (n_q - 1, n_head - 1)} |
                   {(int(a), int(b)) for a, b in zip(rng.integers(0, n_q, n), rng.integers(0, n_head, n))})
+
+
+@pytest.mark.parametrize("D,H,gq,n_q,wide", [(256, 1, 16, 16, False), (256, 4, 4, 64, False), (128, 7, 1, 256, False),
+                                             (128, 8, 4, 64, True), (128, 2, 1, 257, True), (256, 1, 4, 65, True),
+                                             (256, 8, 1, 255, False)])
+def test_which_calls_take_the_32_row_kernel(oracle, lib, dev, D, H, gq, n_q, wide):
+    """More than 256 query rows per KV head, or 256 of at least 8 heads: below, the 16-row kernels are the faster ones. Their
+    result (a call with its output over the queries takes them) has other last bits than the 32-row kernel's."""
+    B = 128 + 4 * 128
+    n_pos = B + 301
+    OL, PL = make_pair(oracle, lib, D, H, 4, 4, 0, 256, 512, n_ctx=4096, n_ubatch=512)
+    view = lib.sjk_layer_view(C.byref(PL))
+    try:
+        K, V = inputs.kv_rows(n_pos, H, D, seed=90)
+        filled_context(lib, dev, OL, view, K, V, B)
+        q = np.random.default_rng(5).standard_normal((n_q, H * gq, D)).astype(np.float32)
+        got = attend(lib, dev, view, B, n_pos, n_pos - n_q, q, 0.0625)
+        dq = dev.put(q)
+        sjk.check(lib.sjk_hip_attend(C.byref(view), B, n_pos, n_pos - n_q, n_q, H * gq, dq, 0.0625, dq, None), "attend over q")
+        same = np.array_equal(dev.get(dq, q.nbytes, np.uint32), got.reshape(-1).view(np.uint32))
+        assert same == (not wide)
+        check_rows(got, oracle_rows(oracle, OL, B, n_pos, q, n_pos - n_q, 0.0625, some_rows(n_q, H * gq, 20, 3)))
+    finally:
+        oracle.layer_free(C.byref(OL))
+        lib.sj_kvarn_layer_free(C.byref(PL))
 
 
 @pytest.mark.parametrize("D", [256, 128])
