@@ -147,9 +147,10 @@ def test_reference_device_test_shape(oracle, lib):
 @pytest.mark.parametrize("bk,bv,body,n_q,D", [(4, 4, 0, 512, 256), (3, 3, 1, 96, 256), (4, 4, 0, 512, 128)],
                          ids=["4/4s-ubatch512", "3/3t-ubatch96", "d128-4/4s-ubatch512"])
 def test_prefill_ubatch(oracle, lib, dev, bk, bv, body, n_q, D):
-    """A prefill ubatch of n_q positions x 16 query heads (GQA 4:1: 4 n_q rows per KV head, many launches of 8
-    tiles) at the end of a context with a sealed body and a tq6_0 tail; the positions of the ubatch are both in
-    the tail and (causally masked) in the body. Sampled rows from every part of the ubatch."""
+    """A prefill ubatch of n_q positions x 16 query heads (GQA 4:1: 4 n_q rows per KV head) at the end of a context with a
+    sealed body and a tq6_0 tail; the positions of the ubatch are both in the tail and (causally masked) in the body.
+    The 4/4 bodies run on the 32-row kernel and, with the output over the queries, in many launches of 8 16-row tiles,
+    as the trellis body does. Sampled rows from every part of the ubatch."""
     H, S, G = 4, 128, 128
     B = S + 12 * G
     n_pos = B + 700
@@ -167,6 +168,11 @@ def test_prefill_ubatch(oracle, lib, dev, bk, bv, body, n_q, D):
                       {(int(a), int(b)) for a, b in zip(rng.integers(0, n_q, 40), rng.integers(0, n_head, 40))})
         worst, l2 = check_rows(got, oracle_rows(oracle, OL, B, n_pos, q, qpos0, 0.0625, rows))
         say("[tiles] ubatch %d: %d rows, worst %.4f of the tolerance, rel L2 %.2e" % (n_q, len(rows), worst, l2))
+        dq = dev.put(q)
+        sjk.check(lib.sjk_hip_attend(C.byref(view), B, n_pos, qpos0, n_q, n_head, dq, 0.0625, dq, None), "attend over q")
+        over = dev.get(dq, q.nbytes, np.float32).reshape(q.shape)
+        worst, l2 = check_rows(over, oracle_rows(oracle, OL, B, n_pos, q, qpos0, 0.0625, rows))
+        say("[tiles] ubatch %d over its queries: worst %.4f of the tolerance, rel L2 %.2e" % (n_q, worst, l2))
     finally:
         oracle.layer_free(C.byref(OL))
         lib.sj_kvarn_layer_free(C.byref(PL))
@@ -544,5 +550,134 @@ def test_prefill_unseen_values_stay_out(oracle, lib, dev, D, staging, sink_type)
             dev.upload(ptr, old, off)
             say("[tiles] prefill D=%d staging %d, %s: %d positions keep their rows" % (D, staging, name, first - qpos0))
     finally:
+        oracle.layer_free(C.byref(OL))
+        lib.sj_kvarn_layer_free(C.byref(PL))
+
+
+@pytest.mark.parametrize("D", [256, 128])
+def test_prefill_batch_on_a_block_pool(oracle, lib, dev, D):
+    """Two sequences of 288 rows per KV head whose records lie in one pool, in another order, behind block tables: one
+    call each, a batch, a batch on one shared workspace and a captured batch's graph, replayed, all give the bits of a
+    call on the layer that holds the records in order. A batch in which one job's output lies over its queries, and one
+    with a workspace below a partial per compute unit, run on the 16-row kernels: the same bits as that job alone."""
+    H, gq, n_q, S, G = 4, 4, 72, 128, 128
+    n_head, scale = H * gq, 1.0 / float(np.sqrt(D))
+    ctx = [(S + 9 * G + 301, 9), (S + 3 * G + 277, 3)]           # (positions, sealed groups)
+    pairs = [make_pair(oracle, lib, D, H, 4, 4, 0, 256, 512, n_ctx=n + 64, n_ubatch=512) for n, _ in ctx]
+    views = [lib.sjk_layer_view(C.byref(PL)) for _, PL in pairs]
+    hip, graph, gexec = dev.hip, C.c_void_p(), C.c_void_p()
+    hip.hipStreamBeginCapture.argtypes = [C.c_void_p, C.c_int]
+    hip.hipStreamEndCapture.argtypes = [C.c_void_p, C.POINTER(C.c_void_p)]
+    hip.hipGraphInstantiate.argtypes = [C.POINTER(C.c_void_p), C.c_void_p, C.c_void_p, C.c_char_p, C.c_size_t]
+    hip.hipGraphLaunch.argtypes = [C.c_void_p, C.c_void_p]
+    hip.hipGraphExecDestroy.argtypes = [C.c_void_p]
+    hip.hipGraphDestroy.argtypes = [C.c_void_p]
+    try:
+        rb, want, want16 = H * pairs[0][0].lay.bytes, [], []
+        order = np.random.default_rng(2).permutation(14)[:12].astype(np.uint32)      # blocks of both, two unused
+        pool = np.zeros((14, rb), np.uint8)
+        q = np.random.default_rng(17).standard_normal((2, n_q, n_head, D)).astype(np.float32)
+        dq, do = [dev.put(q[k]) for k in range(2)], [dev.alloc(q[k].nbytes) for k in range(2)]
+        at, paged = 0, []
+        for k, ((n_pos, ngr), (OL, PL)) in enumerate(zip(ctx, pairs)):
+            K, V = inputs.kv_rows(n_pos, H, D, seed=700 + k)
+            filled_context(lib, dev, OL, views[k], K, V, S + ngr * G)
+            want.append(attend(lib, dev, views[k], S + ngr * G, n_pos, n_pos - n_q, q[k], scale).view(np.uint32))
+            check_rows(want[k].view(np.float32), oracle_rows(oracle, OL, S + ngr * G, n_pos, q[k], n_pos - n_q, scale,
+                                                             some_rows(n_q, n_head, 30, k)))
+            over = dev.put(q[k])
+            sjk.check(lib.sjk_hip_attend(C.byref(views[k]), S + ngr * G, n_pos, n_pos - n_q, n_q, n_head, over, scale, over,
+                                         None), "attend over q")
+            want16.append(dev.get(over, q[k].nbytes, np.uint32).reshape(q[k].shape))
+            assert not np.array_equal(want16[k], want[k])
+            ids = order[at:at + ngr]
+            pool[ids] = dev.get(C.c_void_p(views[k].body), ngr * rb, np.uint8).reshape(ngr, rb)
+            v = sjk.View.from_buffer_copy(bytes(views[k]))
+            v.blocks = dev.put(ids).value
+            paged.append(v)
+            at += ngr
+        d_pool = dev.put(pool)
+        for v in paged:
+            v.body = d_pool.value
+        jobs = (sjk.AttendJob * 2)()
+        for k, (n_pos, ngr) in enumerate(ctx):
+            jobs[k].v, jobs[k].B, jobs[k].N, jobs[k].qpos0 = paged[k], S + ngr * G, n_pos, n_pos - n_q
+            jobs[k].d_q, jobs[k].d_out = dq[k].value, do[k].value
+
+        def outputs():
+            dev.sync()
+            return [dev.get(do[k], q[k].nbytes, np.uint32).reshape(q[k].shape) for k in range(2)]
+
+        def batch(name, expect, stream=None):
+            for k in range(2):
+                dev.upload(do[k], np.full(q[k].shape, np.nan, np.float32))
+            sjk.check(lib.sjk_hip_attend_batch(jobs, 2, n_q, n_head, scale, stream), "attend_batch")
+            for k, x in enumerate(outputs()):
+                assert np.array_equal(x, expect[k]), (name, k)
+
+        for k, (n_pos, ngr) in enumerate(ctx):
+            one = attend(lib, dev, paged[k], S + ngr * G, n_pos, n_pos - n_q, q[k], scale)
+            assert np.array_equal(one.view(np.uint32), want[k]), ("single", k)
+        batch("batch", want)
+        jobs[1].v.work = paged[0].work
+        batch("one workspace", want)
+        stream = dev.stream()
+        dev._ck(hip.hipStreamBeginCapture(stream, 2), "hipStreamBeginCapture")
+        rc = lib.sjk_hip_attend_batch(jobs, 2, n_q, n_head, scale, stream)
+        dev._ck(hip.hipStreamEndCapture(stream, C.byref(graph)), "hipStreamEndCapture")
+        sjk.check(rc, "attend_batch")
+        dev._ck(hip.hipGraphInstantiate(C.byref(gexec), graph, None, None, 0), "hipGraphInstantiate")
+        for _ in range(3):
+            for k in range(2):
+                dev.upload(do[k], np.full(q[k].shape, np.nan, np.float32))
+            dev._ck(hip.hipGraphLaunch(gexec, stream), "hipGraphLaunch")
+            dev._ck(hip.hipStreamSynchronize(stream), "hipStreamSynchronize")
+            for k, x in enumerate(outputs()):
+                assert np.array_equal(x, want[k]), ("graph", k)
+            batch("between replays", want)
+        jobs[1].v.work = paged[1].work
+        # one partial of 32 rows takes two slots of 16 rows and a little more: three quarters of the workspace hold the
+        # 16-row kernels' partials and less than that of every compute unit
+        jobs[1].v.work_bytes = paged[1].work_bytes * 3 // 4
+        single = attend(lib, dev, jobs[1].v, jobs[1].B, jobs[1].N, jobs[1].qpos0, q[1], scale)
+        assert np.array_equal(single.view(np.uint32), want16[1])
+        jobs[1].v.work_bytes = paged[1].work_bytes
+        over = dev.put(q[1])
+        jobs[1].d_q = jobs[1].d_out = over.value
+        sjk.check(lib.sjk_hip_attend_batch(jobs, 2, n_q, n_head, scale, None), "attend_batch")
+        got = [dev.get(do[0], q[0].nbytes, np.float32), dev.get(over, q[1].nbytes, np.float32)]
+        for k, (n_pos, ngr) in enumerate(ctx):       # (tiles of both share launches, so that their split is not the single call's)
+            check_rows(got[k].reshape(q[k].shape), oracle_rows(oracle, pairs[k][0], S + ngr * G, n_pos, q[k], n_pos - n_q,
+                                                               scale, some_rows(n_q, n_head, 30, k)))
+    finally:
+        if gexec.value:
+            hip.hipGraphExecDestroy(gexec)
+        if graph.value:
+            hip.hipGraphDestroy(graph)
+        for OL, PL in pairs:
+            oracle.layer_free(C.byref(OL))
+            lib.sj_kvarn_layer_free(C.byref(PL))
+
+
+@pytest.mark.parametrize("S", [0, 1, 100])
+def test_prefill_any_sink_length(oracle, lib, dev, S):
+    """A hand-built view whose sink is no whole number of steps (or none): the sink's last step ends early, and the tail
+    starts at a position that is no multiple of 16."""
+    D, H, gq, n_q = 256, 2, 4, 72
+    B = S + 5 * 128
+    n_pos = B + 301
+    OL, PL = make_pair(oracle, lib, D, H, 4, 4, 0, 256, 512, n_ctx=4096, n_ubatch=512)
+    view = lib.sjk_layer_view(C.byref(PL))
+    try:
+        view.S = OL.cfg.sink = S
+        K, V = inputs.kv_rows(n_pos, H, D, seed=93)
+        filled_context(lib, dev, OL, view, K, V, B)
+        q = np.random.default_rng(9).standard_normal((n_q, H * gq, D)).astype(np.float32)
+        for qpos0 in (n_pos - n_q, B - 40, max(0, S - 30)):      # rows in the tail, across the body's end, across the sink's
+            got = attend(lib, dev, view, B, n_pos, qpos0, q, 0.0625)
+            worst, l2 = check_rows(got, oracle_rows(oracle, OL, B, n_pos, q, qpos0, 0.0625, some_rows(n_q, H * gq, 30, 7)))
+            say("[tiles] prefill S=%d at %d: worst %.4f of the tolerance, rel L2 %.2e" % (S, qpos0, worst, l2))
+    finally:
+        OL.cfg.sink = 128
         oracle.layer_free(C.byref(OL))
         lib.sj_kvarn_layer_free(C.byref(PL))
