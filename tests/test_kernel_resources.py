@@ -93,13 +93,14 @@ def written(op, text):
 TRANS = ("v_exp_", "v_log_", "v_rcp_", "v_rsq_", "v_sqrt_", "v_sin_", "v_cos_")
 
 
-def asm_mfma_hazards(lines, valu_to_mfma=2, mfma_to_valu=11):
+def asm_mfma_hazards(lines, valu_to_mfma=2, mfma_to_valu=12):
     """Inline-asm VALU instructions next to MFMAs without the wait states between them that the compiler inserts
     only around its own instructions (every instruction is one wait state, s_nop N is N + 1; the scan stops at a
     block label): an MFMA reading a VGPR whose last write was an asm VALU instruction fewer than valu_to_mfma wait
     states before; an asm VALU instruction reading an MFMA result, or writing a register an MFMA reads as its
-    accumulator, fewer than mfma_to_valu wait states after the MFMA (the eight-pass MFMAs of these kernels); an asm
-    VALU instruction reading a transcendental result with no wait state between."""
+    accumulator, fewer than mfma_to_valu wait states after the MFMA (12, what this compiler puts between an eight-pass
+    MFMA and its own VALU instructions on gfx950); an asm VALU instruction reading a transcendental result with no wait
+    state between."""
     ins = parse_asm(lines)
     bad = []
     for k, (op, text, asm) in enumerate(ins):
@@ -138,6 +139,38 @@ def asm_mfma_hazards(lines, valu_to_mfma=2, mfma_to_valu=11):
                 dst -= w
                 waits += int(text2.split()[1]) + 1 if op2 == "s_nop" else 1
     return bad
+
+
+def test_hazard_check_asks_for_what_the_compiler_inserts():
+    def listing(gap, reads):
+        return ["\tv_mfma_f32_32x32x16_f16 v[0:15], v[16:19], v[20:23], v[0:15]", "\ts_nop %d" % (gap - 1), "\t;;#ASMSTART",
+                "\tv_permlane32_swap_b32 v%d, v40" % (3 if reads else 41), "\t;;#ASMEND"]
+    assert asm_mfma_hazards(listing(11, True)) and not asm_mfma_hazards(listing(12, True))
+    assert not asm_mfma_hazards(listing(1, False))
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc is not installed")
+def test_compiler_inserts_no_more_wait_states_than_the_check_asks_for():
+    # an eight-pass MFMA whose result a VALU instruction reads at once
+    src = ("typedef _Float16 h8 __attribute__((ext_vector_type(8)));\ntypedef float f16v __attribute__((ext_vector_type(16)));\n"
+           "__attribute__((global)) void k(const h8 * a, f16v * c, float * o) {\n"
+           "  *o = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0], a[1], *c, 0, 0, 0)[3] * 3.0f;\n}\n")
+    with tempfile.TemporaryDirectory() as d:
+        p, asm = os.path.join(d, "k.hip"), os.path.join(d, "k.s")
+        with open(p, "w") as f:
+            f.write(src)
+        out = subprocess.run([HIPCC] + [x for x in FLAGS if not x.startswith("-Rpass")] + ["-o", asm, p], capture_output=True,
+                             text=True, timeout=600)
+        assert out.returncode == 0, out.stderr[-2000:]
+        with open(asm) as f:
+            ins = [x for lines in kernel_bodies(f.read()).values() for x in parse_asm(lines)]
+    at = next(i for i, x in enumerate(ins) if x[0].startswith("v_mfma"))
+    dst, gap = written(*ins[at][:2]), 0
+    for op, text, _ in ins[at + 1:]:
+        if op.startswith("v_") and vgprs(",".join(operands(text)[1:])) & dst:
+            break
+        gap += int(text.split()[1]) + 1 if op == "s_nop" else 1
+    assert gap <= 12, gap
 
 
 def resources(src):
