@@ -68,6 +68,27 @@ template <int D> struct RecLay4 {
 static_assert(RecLay4<256>::BYTES == R_BYTES && RecLay4<256>::VCH == R_VCH && RecLay4<128>::BYTES == 17920,
               "4/4 record sizes of sj_kvarn.h:792-794 (D = 256, 128)");
 
+// Trellis pair tables: entry e (6 + 2B bits of a channel stream, oldest bit first) holds the fp16
+// codebook values of the two windows it contains, cb[e & (2^(6+B) - 1)] | cb[e >> B] << 16.
+template <int B> struct PairTab { uint32_t v[1 << (6 + 2 * B)]; };
+template <int B, int NC>
+constexpr PairTab<B> make_pairs(const uint16_t (&cb)[NC]) {
+    PairTab<B> t{};
+    for (uint32_t e = 0; e < (1u << (6 + 2 * B)); ++e)
+        t.v[e] = (uint32_t) cb[e & ((1u << (6 + B)) - 1u)] | ((uint32_t) cb[e >> B] << 16);
+    return t;
+}
+constexpr uint16_t k_cb3k[512] = SJK_CB3_K_INIT, k_cb3v[512] = SJK_CB3_V_INIT;
+constexpr uint16_t k_cb2k[256] = SJK_CB2_K_INIT, k_cb2v[256] = SJK_CB2_V_INIT;
+static __device__ const PairTab<3> g_pair3k = make_pairs<3>(k_cb3k);
+static __device__ const PairTab<3> g_pair3v = make_pairs<3>(k_cb3v);
+static __device__ const PairTab<2> g_pair2k = make_pairs<2>(k_cb2k);
+static __device__ const PairTab<2> g_pair2v = make_pairs<2>(k_cb2v);
+template <int B, bool IS_V> SJK_DEV const uint32_t * pair_tab() {
+    if (B == 3) return IS_V ? g_pair3v.v : g_pair3k.v;
+    return IS_V ? g_pair2v.v : g_pair2k.v;
+}
+
 struct A3Args {
     sjk_hip_view v;
     uint32_t N, qpos0;

@@ -63,6 +63,11 @@ SJK_DEV void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// v of the lane that the DPP control names (in the same 16-lane row)
+template <int CTRL> SJK_DEV float dpp(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+}
+
 // Row exchange between two registers: v_permlane16_swap_b32 swaps the odd 16-lane rows of x with the even
 // rows of y, v_permlane32_swap_b32 the upper 32 lanes of x with the lower 32 of y (no LDS round trip, unlike
 // a lane shuffle). Written out as asm because this toolchain's builtin returns the first register for both

@@ -119,14 +119,11 @@ SJK_DEV float half_max(float v) {
     return fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
 }
 // the largest over 16 lanes (a DPP row)
-template <int ROR> SJK_DEV float ror(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + ROR, 0xF, 0xF, false));
-}
 SJK_DEV float row_max(float v) {
-    v = fmaxf(v, ror<8>(v));
-    v = fmaxf(v, ror<4>(v));
-    v = fmaxf(v, ror<2>(v));
-    return fmaxf(v, ror<1>(v));
+    v = fmaxf(v, dpp<0x128>(v));                 // row_ror 8, 4, 2, 1
+    v = fmaxf(v, dpp<0x124>(v));
+    v = fmaxf(v, dpp<0x122>(v));
+    return fmaxf(v, dpp<0x121>(v));
 }
 
 // the context of a tile of query rows, whose last row is row `last`
@@ -1002,10 +999,6 @@ template <int D> __global__ __launch_bounds__(PF_NT) void prefill_combine(const 
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[i] = y[i] * inv;
 }
-
-}  // namespace sjk
-
-namespace sjk {
 
 // The kernel takes 4/4 bodies whose workspace holds one partial per CU and whose rows are not written where another
 // workgroup still reads queries (a call with out over q takes the 16-row kernels, which write after all reads).

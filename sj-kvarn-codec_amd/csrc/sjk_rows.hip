@@ -77,10 +77,6 @@ struct RowBatch {
 
 static_assert(sizeof(RowBatch) <= 4096, "the job table travels in the kernel arguments");
 
-template <int CTRL> SJK_DEV float dpp(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
-}
-
 // Hadamard of one row held V values per lane (sj_kvarn.h:735-752): stages h < V inside the lane, stages h >= V
 // between lanes l and l ^ (h / V) (the lower partner keeps a + b, the upper a - b, a = the lower value), then one
 // multiply by 1/sqrt(D). XN: the host's NaN rule (a row holding an infinity or a NaN).

@@ -387,8 +387,6 @@ SJK_DEV void col_scales(const SealArgs & a, SealLds & s, uint8_t * rec) {
 // trellis
 // ------------------------------------------------------------------------------------------------
 
-SJK_DEV float readlane_f(float x, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane)); }
-
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 // p = 2 p + (bit `lane` of m), one instruction. m must come from the scalar unit (a mask straight from a vector
