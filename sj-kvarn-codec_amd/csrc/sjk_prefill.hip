@@ -24,10 +24,10 @@
 // channels are 2^20 apart and up to 1.1x further off than now with Kscale near 2^-9.
 //
 // What bounds it (D = 256): vector issue. A record is 128 + 64 products of 32 cycles, 6,100 cycles of a SIMD's matrix
-// core, and about 2,300 vector instructions, 10,000 cycles at their measured 2.5-5 each; 32 staged positions 96
-// products and 1,900 instructions. Two wavefronts per SIMD (O alone is 128 of their 256 registers) overlap the two only in
-// part. 512 positions x 16 heads at 32K, D = 256: 660 us against 1,322 us with the 16-row kernels (5.5K staged
-// positions; 275 GFLOP of products at one pass, 0.41 PFLOP/s).
+// core, and about 2,300 vector instructions; 32 staged positions 96 products and 1,050 (tq6_0 rows). Two wavefronts per SIMD
+// (O alone is 128 of their 256 registers) overlap the two only in part: counted over a call, a SIMD issues vector
+// instructions 62% of the time and its matrix core is busy 35%. 512 positions x 16 heads at 32K, D = 256: 640 us against
+// 1,315 us with the 16-row kernels (6.8K staged positions; 273 GFLOP of products at one pass, 0.43 PFLOP/s).
 #include "sjk_mfma.h"
 
 #include <type_traits>
@@ -41,8 +41,8 @@ constexpr int PF_CH = 32;                        // staged positions per step
 constexpr int PF_MSTR = 68;                      // floats per query row of a merge slice (64 channels, 16-byte rows)
 constexpr int PF_WAVE = PF_CH * 200;             // LDS bytes per wavefront: staged V rows and K norms
 
-// cost of 32 staged positions and of a sealed record: 3 : 4 was the fastest; 7 : 10 took 2% longer, 2 : 3 1.5% and 5 : 9 8% on
-// the 32K ubatch above
+// cost of 32 staged positions and of a sealed record: 3 : 4 was the fastest (7 : 10 took 0-1% longer, 2 : 3 1-3%, 5 : 9 5-8%
+// on 512-position ubatches at 16K and 32K, D = 128 and 256)
 constexpr int PF_COST_CH = 3, PF_COST_REC = 4;
 
 // Calls with fewer query rows per KV head take the 16-row kernels. Past 256 rows, where those take a third launch, this

@@ -17,10 +17,11 @@ namespace sjk {
 // Wavefronts (rows) per workgroup. A walk takes 32 16-byte LDS reads whatever the number of lanes that use it, so
 // with a walk per row (ROW_WAVES) a large tq6_0 call is bound by them; with the walks of a workgroup's rows in one
 // wavefront's lanes (ROW_WAVES_BIG) the others wait at a barrier, which costs a small call its latency. Appends at
-// D = 128 / 256, walk per row against one wavefront's: 2,048 rows 4.7 / 5.2 against 5.8 / 6.8 us, 4,096 rows 6.1 / 7.0
-// against 6.0 / 6.9, 8,192 rows 8.7 / 10.7 against 7.5 / 9.1: the line is at a large workgroup per CU. Rows that are no
-// tq6_0 leave before the walks; among them the small workgroups are the faster at every size (8,192 fp16 rows 4.4 /
-// 5.1 against 5.1 / 6.0 us, with the walks 9.0 / 11.0).
+// D = 128 / 256, walk per row against one wavefront's: 2,048 rows 4.5 / 4.9 against 5.6 / 6.4 us, 4,096 rows 5.8 / 6.4
+// against 5.8 / 6.5, 8,192 rows 8.2 / 9.5 against 7.4 / 8.7, 16,384 rows 13.5 / 15.9 against 12.4 / 15.1: the line is
+// at a large workgroup per CU (past it a second, partly filled round of them costs 6,144 rows 2-6%: 7.1 / 8.0 against
+// 7.2 / 8.5). Rows that are no tq6_0 leave before the walks; among them the small workgroups are the faster at every size
+// (8,192 fp16 rows 4.1 / 5.0 against 4.9 / 6.0 us, with the walks 9.0 / 11.0).
 constexpr int ROW_WAVES = 4, ROW_WAVES_BIG = 16;
 enum { OUT_F32 = 0, OUT_F16 = 1, OUT_TQ6 = 2 };
 
