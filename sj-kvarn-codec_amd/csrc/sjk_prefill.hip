@@ -1001,13 +1001,15 @@ template <int D> __global__ __launch_bounds__(PF_NT) void prefill_combine(const 
 }
 
 // The kernel takes 4/4 bodies whose workspace holds one partial per CU and whose rows are not written where another
-// workgroup still reads queries (a call with out over q takes the 16-row kernels, which write after all reads).
+// workgroup still reads queries (a call with out over q takes the 16-row kernels, which write after all reads). Staged
+// tq6_0 rows are copied to LDS by words, so that a hand-built view with them at odd halves keeps the 16-row kernels too.
 bool sjk_prefill_takes(const sjk_hip_view & v, int body, int n_q, int n_head, const float * d_q, const float * d_out) {
     const size_t row = (size_t) n_q * (size_t) n_head * (size_t) v.lay.D, W = (size_t) n_cus(), sf = ws_slot_floats(v.lay.D);
     const int rows = n_q * (n_head / v.n_head_kv);
     if (rows < PF_MIN_ROWS || (rows == PF_MIN_ROWS && v.n_head_kv < PF_MIN_ROWS_HEADS)) return false;
     if (body != 44 || v.work_bytes < WS_PLAN_BYTES + ws_stage_bytes(v.lay.D, v.n_head_kv)) return false;
     if (d_q < d_out + row && d_out < d_q + row) return false;
+    if (v.staging != SJKVARN_STAGING_F16 && (((uintptr_t) v.sink | (uintptr_t) v.ring) & 3u)) return false;
     return W * PF_ROWS * (size_t) v.lay.D + W * PF_ROWS * 4 <= ws_part_slots(v) * sf;
 }
 
