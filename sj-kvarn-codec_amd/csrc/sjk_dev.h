@@ -52,8 +52,8 @@ SJK_DEV float f16_to_f32(uint16_t h) {
     return sign ? -v : v;
 }
 
-// half -> float on the hardware converter: exact for every half except that it quiets signalling
-// NaNs; used where only values matter (attention), never for bytes that are compared
+// half -> float on the hardware converter: exact for every half except that it quiets signalling NaNs; used where only
+// values matter (attention) or only a NaN's sign does (decoded rows, see dequant_x), never for other bytes
 SJK_DEV float f16_to_f32_fast(uint16_t h) { return (float) __builtin_bit_cast(_Float16, h); }
 
 // LDS written by lanes of this wavefront is read by others of it
