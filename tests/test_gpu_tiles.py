@@ -681,3 +681,36 @@ def test_prefill_any_sink_length(oracle, lib, dev, S):
         OL.cfg.sink = 128
         oracle.layer_free(C.byref(OL))
         lib.sj_kvarn_layer_free(C.byref(PL))
+
+
+@pytest.mark.parametrize("D,staging", [(128, 0), (256, 0), (256, 1)])
+def test_prefill_staged_rows_against_float64(oracle, lib, dev, D, staging):
+    """All positions staged, so that only 32-bit sums and split operands are in the path (about 4e-7): the 32-row kernel is
+    no further from float64 attention over the same rows than the 16-row kernels (the call with its output over the
+    queries). One KV head, every row."""
+    H, gq, n_q, n_pos, S = 2, 4, 300, 4000, 128
+    OL, PL = make_pair(oracle, lib, D, H, 4, 4, 0, 4096, 8192, n_ctx=8192, n_ubatch=512, staging=staging)
+    view = lib.sjk_layer_view(C.byref(PL))
+    try:
+        K, V = inputs.kv_rows(n_pos, H, D, seed=94, outlier_scale=1.0)
+        filled_context(lib, dev, OL, view, K, V, S)
+        q = np.random.default_rng(13).standard_normal((n_q, H * gq, D)).astype(np.float32)
+        scale, qpos0 = 1.0 / float(np.sqrt(D)), n_pos - n_q
+        got = attend(lib, dev, view, S, n_pos, qpos0, q, scale)
+        dq = dev.put(q)
+        sjk.check(lib.sjk_hip_attend(C.byref(view), S, n_pos, qpos0, n_q, H * gq, dq, scale, dq, None), "attend over q")
+        over = dev.get(dq, q.nbytes, np.float32).reshape(q.shape)
+        k64, v64 = (np.zeros((n_pos, D), np.float32) for _ in range(2))
+        for p in range(n_pos):
+            oracle.layer_kv_row(C.byref(OL), S, p, 0, cabi.ptr(k64[p], cabi.f32p), cabi.ptr(v64[p], cabi.f32p))
+        rows = q[:, :gq].reshape(-1, D).astype(np.float64)
+        sc = rows @ k64.astype(np.float64).T * scale
+        sc[np.arange(n_pos)[None, :] > (qpos0 + np.arange(n_q).repeat(gq))[:, None]] = -np.inf
+        pw = np.exp(sc - sc.max(axis=1, keepdims=True))
+        want = (pw @ v64.astype(np.float64)) / pw.sum(axis=1, keepdims=True)
+        err = [float(np.linalg.norm(x[:, :gq].reshape(-1, D) - want) / np.linalg.norm(want)) for x in (got, over)]
+        say("[tiles] staged rows D=%d staging %d: error against float64 %.3e, 16-row kernels %.3e" % (D, staging, *err))
+        assert err[0] <= err[1]
+    finally:
+        oracle.layer_free(C.byref(OL))
+        lib.sj_kvarn_layer_free(C.byref(PL))
