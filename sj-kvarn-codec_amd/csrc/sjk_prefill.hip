@@ -20,8 +20,9 @@
 // hi + lo parts (times a power of two per row, so that a large row does not overflow and a small one does not lose its low
 // part), a tq6_0 value as the hi + lo parts of its centroid, the K block norm multiplies the fp32 sum of its block, the V
 // block norm the weight P, which is split hi + lo: three products each. Error against float64 at 7K-20K positions 0.91-1.0 of
-// the 16-row kernels' on values of unit variance, 0.73-1.06 on queries, keys or zero points 2^5-2^10 off. Q' from a query cut to fp16 parts first took 1% less time, but was off by 8e-3 on rows whose
-// channels are 2^20 apart and up to 1.1x further off than now with Kscale near 2^-9.
+// the 16-row kernels' on values of unit variance, 0.73-1.06 on queries, keys or zero points 2^5-2^10 off. Q' from a query
+// cut to fp16 parts first took 1% less time, but was off by 8e-3 on rows whose channels are 2^20 apart and up to 1.1x
+// further off than now with Kscale near 2^-9.
 //
 // What bounds it (D = 256): vector issue. A record is 128 + 64 products of 32 cycles, 6,100 cycles of a SIMD's matrix
 // core, and about 2,300 vector instructions; 32 staged positions 96 products and 1,050 (tq6_0 rows). Two wavefronts per SIMD
