@@ -27,8 +27,9 @@
 // What bounds it (D = 256): vector issue. A record is 128 + 64 products of 32 cycles, 6,100 cycles of a SIMD's matrix
 // core, and about 2,300 vector instructions; 32 staged positions 96 products and 1,050 (tq6_0 rows). Two wavefronts per SIMD
 // (O alone is 128 of their 256 registers) overlap the two only in part: counted over a call, a SIMD issues vector
-// instructions 62% of the time and its matrix core is busy 35%. 512 positions x 16 heads at 32K, D = 256: 640 us against
-// 1,315 us with the 16-row kernels (6.8K staged positions; 273 GFLOP of products at one pass, 0.43 PFLOP/s).
+// instructions 62% of the time and its matrix core is busy 35%. 512 positions x 16 heads at 32K, D = 256: 640-665 us by card
+// against 1,315-1,330 us with the 16-row kernels (6.8K staged positions; 273 GFLOP of products at one pass, 0.41-0.43
+// PFLOP/s).
 #include "sjk_mfma.h"
 
 #include <type_traits>
